@@ -1362,7 +1362,7 @@ __global__ void __launch_bounds__(512) attn_prefill_ws_kernel(const AttnArgs a) 
       // the gathers of tile t + 2 into buffer (t + 2) % NBUF (tile t - 2's: every read of it ended before B0; its
       // pointers were resolved in iteration t - 1); then the V fragments of tile t - 1
       // (near the end the gathers of tiles past the row land in buffers no wave reads again, from row pointers
-      // left by earlier tiles: no branch per load; E1 waits for them before the buffers take the output)
+      // left by earlier tiles: no branch per load; they are waited for before E1)
       const int tp = t - 2;
       sources(t + 2);
       const uint16_t* vrow = ktile + ((t + NBUF - 1) % NBUF) * TILE_ELEMS + vj * DQK + ((l16 & 1) << 2);
@@ -1417,6 +1417,9 @@ __global__ void __launch_bounds__(512) attn_prefill_ws_kernel(const AttnArgs a) 
       }
       PF_TS(11, 256);
     }
+    // the gathers past the row have landed (__syncthreads is a workgroup fence: it waits for LDS operations, not for
+    // these direct-to-LDS loads, which would overwrite the staged output)
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
     __syncthreads();  // E1: every PV wave is past its last V read, so the tile buffers can take the output
 #pragma unroll
     for (int b = 0; b < 4; ++b)

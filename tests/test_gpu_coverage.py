@@ -56,6 +56,43 @@ def _rope_tables(rd, n):
 
 
 # ------------------------------------------------------------------------------------------ many-row attention
+@pytest.mark.parametrize("dqk,R,k,n", [(576, 32, 2048, 6000), (576, 48, 300, 250), (512, 24, 512, 9000)])
+def test_sattn2_many_rows_unit_scale(dqk, R, k, n):
+    """The 64-head kernel at values of unit size against a float64 softmax, three launches bit-equal: gathers still in
+    flight when the output is staged would show in single elements.  Rows end in empty entries as short contexts do.
+    Bound per output row: bf16 probabilities, partials and result, 2^-9 each, and their sums: 2^-7."""
+    import dsv41_amd
+    g = torch.Generator(device=DEV).manual_seed(7)
+    H, dv, win = 64, 512, 128
+    rn = lambda *s: torch.randn(*s, generator=g, device=DEV).to(torch.bfloat16)  # noqa: E731
+    q, ring, ckv = rn(R, 1, H, dqk), rn(R, win, dqk), rn(R, n, dqk)
+    sink = torch.randn(H, generator=g, device=DEV)
+    idx = torch.rand(R, n, generator=g, device=DEV).argsort(-1)[:, :k].to(torch.int32)
+    if k > n:
+        idx = torch.cat([idx, torch.full((R, k - n), -1, device=DEV, dtype=torch.int32)], -1)
+    for r in range(R):  # ever shorter contexts: -1 tails
+        idx[r, k - (r * k) // (R + 4):] = -1
+    pos = torch.arange(R, device=DEV) + 5000
+    seq = torch.arange(R, device=DEV)
+    cos, sin = (x.to(DEV) for x in _rope_tables(64, 8192))
+    rd = 64 if dqk == 512 else 0
+    got = [dsv41_amd.sattn2(q, ring, ckv, idx.unsqueeze(1), pos, sink, cos, sin, rd, dqk ** -0.5, seq, pos, d_v=dv)
+           for _ in range(3)]
+    assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
+    for r in range(R):
+        sel = idx[r][idx[r] >= 0].long()
+        rows = torch.cat([ring[r], ckv[r, sel]]).double()
+        lg = q[r, 0].double() @ rows.t() * dqk ** -0.5
+        e = torch.exp(lg - lg.amax(-1, keepdim=True))
+        want = e @ rows[:, :dv] / (e.sum(-1, keepdim=True) + torch.exp(sink.double()[:, None] - lg.amax(-1, keepdim=True)))
+        if rd:  # inverse rope on the last rd columns
+            c, s = cos[pos[r]].double(), -sin[pos[r]].double()
+            a, b = want[:, -rd::2].clone(), want[:, -rd + 1::2].clone()
+            want[:, -rd::2], want[:, -rd + 1::2] = a * c - b * s, a * s + b * c
+        rel = (got[0][r, 0].double() - want).norm(dim=-1) / want.norm(dim=-1)
+        assert rel.max() < 2 ** -7, (r, float(rel.max()))
+
+
 @pytest.mark.parametrize("nsplit", [0, 3, 1])
 def test_sattn2_mla_48_rows_ragged_drafts(nsplit):
     """C5's attention shape (dsv41/fused2.py:334-446): 8 ragged slots x (1 + 5 MTP drafts) = 48 rows, absorbed MLA

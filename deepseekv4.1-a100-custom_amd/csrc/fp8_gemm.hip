@@ -5,7 +5,8 @@
 // permuted (position p holds k = 16 (p / 16) + kPermK[p % 16]); S is E8M0 per [32 n x 32 k] block.  row(m, n) = m,
 // or with group_cols > 0 (block-diagonal o-projection) m * (N / group_cols) + n / group_cols.
 //
-// A weight stream: every weight byte is read once per 64 output rows.  Workgroup = 4 waves x 16 columns (64
+// Up to 16 rows, and where the tile kernels (fp8_tile.h) do not apply (x rows not 16-byte aligned, K > 16384), a
+// weight stream: every weight byte is read once per 64 output rows.  Workgroup = 4 waves x 16 columns (64
 // columns) over a K slice; a lane loads 16 weight bytes (one 16-k group, inside one scale block) per 64-k window and
 // converts them to bf16 with the block scale applied by the hardware (v_cvt_scalef32_pk_bf16_fp8: exact, the e4m3
 // values times a power of two); the x slice is staged in LDS in the weights' byte order, so a bf16 MFMA (16 rows x
@@ -16,6 +17,7 @@
 // (16 columns, 16 waves over the whole K) and the vector one (a few columns per workgroup, fp32 VALU dot products);
 // the plan picks by rows and columns, from measurements.  All three are deterministic.
 #include "common.h"
+#include "fp8_tile.h"
 #include "rowop.h"
 
 namespace {
@@ -493,6 +495,114 @@ GemmPlan gemm_plan(int M, int N, int K, bool narrow_ok) {
   return p;
 }
 
+// ---- tile kernels (fp8_tile.h): launch shapes and the choice between them
+struct TileShape {
+  int bm, bn, ku, wgs;  // rows, columns, units per stage, workgroups a CU holds
+  float t1, t2, fix;    // us per 64 k with one / two workgroups on a CU, and per workgroup (fill, epilogue)
+};
+// The times are measured ones (2048 to 24 rows over the projections' shapes).  The 256-row shapes slow down as the
+// grid fills the chip (power): t1 with one CU in hand, t2 with all.
+constexpr TileShape kTiles[] = {
+    {32, 64, 4, 1, 0.235f, 0.0f, 2.4f},   {32, 128, 4, 1, 0.30f, 0.0f, 2.4f}, {64, 64, 2, 2, 0.30f, 0.48f, 2.0f},
+    {64, 128, 1, 2, 0.43f, 0.66f, 2.0f},  {128, 128, 1, 2, 0.62f, 1.05f, 2.5f}, {192, 256, 1, 1, 1.03f, 1.18f, 6.0f},
+    {256, 256, 1, 1, 1.27f, 1.68f, 8.0f}};
+constexpr int kTileShapes = sizeof(kTiles) / sizeof(kTiles[0]);
+// Columns up to which the sums stay the streaming kernel's bit for bit: the kv latents (512 columns), whose rows go on
+// to the fp8 grid, where a last bit of a sum becomes a whole step.  Cost at 5120 k, us, against the fastest plan and
+// the stream: 100 rows 11.7 (9.5, 84), 800 23.1 (17.1, 555), 2048 28.6 (25.5, 1425), 3000 46.4 (35.8, 2100).
+constexpr int kTileSameN = 512;
+constexpr int kTileMinM = 17;             // up to 16 rows the streaming kernels read the weights once as well
+constexpr long kTilePartMax = 64l << 20;  // bytes of K-slice partials
+
+struct TilePlan {
+  int shape, splits;  // shape < 0: not for the tile kernels
+  int chain;          // units of an MFMA chain, also of a K slice when same
+  bool same;
+};
+
+// The shape and K slices of the least estimated time: rounds of workgroups over 256 CUs, times their stages, plus the
+// slices' partials written and read and the launch that sums them.  f32: a caller that takes the fp32 sums gets the
+// shapes that keep their chains short.
+TilePlan tile_plan(int M, int N, int K, int group_cols, bool f32) {
+  TilePlan best{-1, 1, 0, false};
+  if (M < kTileMinM || K > kTileMaxK) return best;
+  const int chain = gemm_plan(M, N, K, false).kslice / 64;
+  const bool same = N <= kTileSameN;
+  float tbest = 0.0f;
+  for (int c = 0; c < kTileShapes; ++c) {
+    const TileShape& t = kTiles[c];
+    if (K % (64 * t.ku) || (group_cols > 0 && group_cols % t.bn) || ((f32 || same) && t.bm > 128) ||
+        (t.bm > 128 && M <= 128) || (same && (c == 1 || chain % t.ku)))
+      continue;
+    const long tiles = (long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+    const int stages = K / (64 * t.ku), slices = (K / 64 + chain - 1) / chain;
+    for (int s = 1; s <= (same ? slices : 8) && (t.bm <= 128 || s == 1); s = same ? (s < slices ? slices : s + 1) : 2 * s) {
+      if (s > 1 && !same && (stages < 2 * s || (long)s * M * N * 4 > kTilePartMax || tiles * (s / 2) >= 512)) break;
+      const long wg = tiles * s, percu = (wg + 255) / 256, rounds = (percu + t.wgs - 1) / t.wgs;
+      const float units = (float)((stages + s - 1) / s * t.ku);
+      const float fill = wg < 256 ? wg / 256.0f : 1.0f;
+      const float u = t.wgs == 1 ? (t.t2 > 0.0f ? t.t1 + (t.t2 - t.t1) * fill : t.t1) : percu == 1 ? t.t1 : t.t2;
+      float us = rounds * (t.fix + units * u);
+      if (s > 1) us += 3.0f + (float)s * M * N * 8.0f / 4e6f;
+      if (best.shape < 0 || us < tbest) {
+        best = TilePlan{c, s, chain < t.ku ? t.ku : chain / t.ku * t.ku, same};
+        tbest = us;
+      }
+    }
+  }
+  return best;
+}
+
+// A tile's x rows are addressed by 32-bit byte offsets from its first.
+bool tile_rows_ok(long ldx, long xr_mul) { return 256 * xr_mul * ldx * 2 < (1l << 31); }
+
+long tile_part_bytes(int M, int N, const TilePlan& p) {
+  return p.shape >= 0 && p.splits > 1 ? (long)p.splits * M * ((N + 3) / 4 * 4) * 4 : 0;
+}
+
+// One launch shape; refuses what its addressing does not take.
+template <int C, int WM, int WN, int NBUF, bool PP, bool SAME>
+int tile_run(TileArgs a, const TilePlan& p, hipStream_t st) {
+  constexpr int BM = kTiles[C].bm, BN = kTiles[C].bn, KU = kTiles[C].ku;
+  if (a.K % (64 * KU) || a.K > kTileMaxK || (a.group_cols > 0 && a.group_cols % BN) || p.chain % KU ||
+      BM * (long)a.xr_mul * a.ldx * 2 >= (1l << 31))
+    return (int)hipErrorInvalidValue;
+  const int stages = a.K / (64 * KU);
+  a.chain = p.chain;
+  a.kslice = SAME && p.splits > 1 ? p.chain : (stages + p.splits - 1) / p.splits * KU;
+  a.splits = (stages * KU + a.kslice - 1) / a.kslice;
+  if (a.splits > p.splits) return (int)hipErrorInvalidValue;
+  a.mtiles = (a.M + BM - 1) / BM;
+  a.ntiles = (a.N + BN - 1) / BN;
+  const long tiles = ((long)a.mtiles * a.ntiles + kXcds - 1) / kXcds * kXcds;
+  if (tiles >= (1l << 31)) return (int)hipErrorInvalidValue;
+  fp8_tile_kernel<BM, BN, WM, WN, NBUF, KU, PP, SAME>
+      <<<dim3((unsigned)tiles, a.splits), 64 * WM * WN, 0, st>>>(a);
+  DSV41_CHECK_LAUNCH();
+  if (a.splits > 1) {
+    tile_sum_kernel<<<dim3((unsigned)((a.ldp / 4 * a.M + 255) / 256)), 256, 0, st>>>(a);
+    DSV41_CHECK_LAUNCH();
+  }
+  return 0;
+}
+
+int tile_launch(const TileArgs& a, const TilePlan& p, hipStream_t st) {
+  switch (p.shape + 16 * p.same) {
+    case 0: return tile_run<0, 1, 2, 4, false, false>(a, p, st);
+    case 1: return tile_run<1, 1, 4, 3, false, false>(a, p, st);
+    case 2: return tile_run<2, 2, 2, 3, false, false>(a, p, st);
+    case 3: return tile_run<3, 1, 4, 4, false, false>(a, p, st);
+    case 4: return tile_run<4, 2, 2, 3, false, false>(a, p, st);
+    case 5: return tile_run<5, 2, 4, 3, true, false>(a, p, st);
+    case 6: return tile_run<6, 2, 4, 3, true, false>(a, p, st);
+    case 16: return tile_run<0, 1, 2, 4, false, true>(a, p, st);
+    case 18: return tile_run<2, 2, 2, 3, false, true>(a, p, st);
+    case 19: return tile_run<3, 1, 4, 4, false, true>(a, p, st);
+    case 20: return tile_run<4, 2, 2, 3, false, true>(a, p, st);
+  }
+  return (int)hipErrorInvalidValue;
+}
+
 }  // namespace
 
 extern "C" {
@@ -500,8 +610,18 @@ extern "C" {
 long dsv41_fp8_gemm_workspace_bytes(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   const GemmPlan p = gemm_plan(M, N, K, false);  // the largest need: the narrow kernel uses none
-  if (p.splits == 1) return 0;
-  return (long)p.ctiles * 4 + 12 + (long)p.splits * 16 * p.MT * N * 4;  // counters, pad, partials
+  long part = p.splits == 1 ? 0 : (long)p.splits * 16 * p.MT * N * 4;
+  for (int f = 0; f < 6; ++f) {  // (every class of group_cols the plan tells apart, with and without the fp32 result)
+    const long t = tile_part_bytes(M, N, tile_plan(M, N, K, f % 3 * kGemmCols, f >= 3));
+    part = t > part ? t : part;
+  }
+  return part ? (long)p.ctiles * 4 + 12 + part : 0;  // counters, pad, partials
+}
+
+int dsv41_fp8_gemm_tiled(int M, int N, int K, int group_cols) {
+  return M > 0 && N > 0 && K > 0 && K % 64 == 0 && tile_rows_ok(K, group_cols > 0 ? N / group_cols : 1) &&
+         tile_plan(M, N, K, group_cols, false).shape >= 0 &&
+         tile_plan(M, N, K, group_cols, true).shape >= 0;
 }
 
 int dsv41_fp8_gemm(const void* x, long ldx, const void* w8, const void* s8, int M, int N, int K, int Kc,
@@ -511,6 +631,32 @@ int dsv41_fp8_gemm(const void* x, long ldx, const void* w8, const void* s8, int 
       ((uintptr_t)x & 3) != 0 || ((uintptr_t)w8 & 15) != 0 ||
       (group_cols > 0 && (group_cols % kGemmCols != 0 || N % group_cols != 0)) || group_cols < 0)
     return (int)hipErrorInvalidValue;
+  const long part0 = ((long)((N + kGemmCols - 1) / kGemmCols) * 4 + 15) / 16 * 16;  // the partials' place in ws
+  const long xr_mul = group_cols > 0 ? N / group_cols : 1;
+  if (((uintptr_t)x & 15) == 0 && ldx % 8 == 0 && tile_rows_ok(ldx, xr_mul)) {
+    const TilePlan t = tile_plan(M, N, K, group_cols, out_f32 != nullptr);
+    const long need = tile_part_bytes(M, N, t);
+    if (t.shape >= 0 && (need == 0 || (ws && ws_bytes >= part0 + need && ((uintptr_t)ws & 15) == 0))) {
+      TileArgs a{};
+      a.x = (const uint16_t*)x;
+      a.ldx = ldx;
+      a.w8 = (const uint8_t*)w8;
+      a.s8 = (const uint8_t*)s8;
+      a.M = M;
+      a.N = N;
+      a.K = K;
+      a.Kc = Kc;
+      a.group_cols = group_cols;
+      a.xr_mul = (int)xr_mul;
+      a.out = (uint16_t*)out;
+      a.ldo = ldo;
+      a.outf = out_f32;
+      a.vec = ldo % 4 == 0 && ((uintptr_t)out & 7) == 0 && ((uintptr_t)out_f32 & 15) == 0;
+      a.part = need ? (float*)((char*)ws + part0) : nullptr;
+      a.ldp = (N + 3) / 4 * 4;
+      return tile_launch(a, t, (hipStream_t)stream);
+    }
+  }
   // the narrow kernel loads x in 16-byte units
   const GemmPlan p = gemm_plan(M, N, K, ((uintptr_t)x & 15) == 0 && ldx % 8 == 0);
   if (p.splits > 1 && (!ws || ws_bytes < dsv41_fp8_gemm_workspace_bytes(M, N, K))) return (int)hipErrorInvalidValue;

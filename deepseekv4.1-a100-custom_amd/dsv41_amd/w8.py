@@ -87,7 +87,13 @@ def fp8_gemm_tc(x: torch.Tensor, w8: torch.Tensor, s8: torch.Tensor, group_cols:
     Mo = xc.shape[0] // (N // group_cols) if group_cols else xc.shape[0]
     out = torch.empty(Mo, N, device=dev, dtype=torch.bfloat16)
     outf = torch.empty(Mo, N, device=dev, dtype=torch.float32) if out_dtype == torch.float32 else None
-    ws, n = _workspace(dev, Mo, N, K)
+    if Mo > 16 and lib().dsv41_fp8_gemm_tiled(Mo, N, K, int(group_cols)):
+        if xc.data_ptr() % 16:  # (the tile kernels load x in 16-byte units)
+            xc = xc.clone()
+        n = lib().dsv41_fp8_gemm_workspace_bytes(Mo, N, K)  # no counters: a workspace of this call alone
+        ws = torch.empty(n, dtype=torch.uint8, device=dev) if n > 0 else None
+    else:
+        ws, n = _workspace(dev, Mo, N, K)
     call("dsv41_fp8_gemm", ptr(xc), K, ptr(w8), ptr(s8), Mo, N, K, s8.shape[1], int(group_cols), ptr(out), N,
          ptr(outf), ptr(ws), n, stream(dev))
     return outf if outf is not None else out

@@ -282,12 +282,16 @@ int dsv41_index_keys_decode(const void* k8, const float* ks, long n_rows, void* 
  * once per shape: every launch leaves its arrival counters at zero (launches sharing it must be stream-ordered). */
 long dsv41_fp8_gemm_workspace_bytes(int M, int N, int K);
 
+/* 1 when dsv41_fp8_gemm runs these sizes, with x contiguous and 16-byte aligned, on the tile kernels: their workspace holds no counters, so it needs neither zeroing nor a life beyond the call. */
+int dsv41_fp8_gemm_tiled(int M, int N, int K, int group_cols);
+
 /* fp8_gemm_tc / fp8_gemv_m1 (dsv41/cukern.py:116-200; weight format dsv41/w8.py:19-60): out[m, n] =
  * sum_k x[row(m, n), k] * e4m3(w8[n, k]) * 2^(s8[n / 32, k / 32] - 127), bf16 x (row stride ldx), fp32
  * accumulation, bf16 out [M, ldo] (and fp32 out_f32 [M, ldo] when not null).  w8: e4m3 bits [N, K] with every 16-k
  * group in the PERM_K byte order; s8: E8M0 [ceil(N / 32), Kc], Kc >= K / 32.  row(m, n) = m, or with group_cols > 0
  * (block-diagonal, dsv41/w8.py oproj_a) m * (N / group_cols) + n / group_cols.  K % 64 == 0; group_cols % 64 == 0;
- * x 4-byte and w8 16-byte aligned.  The weights stream once per 64 rows of M.  With x 16-byte aligned and ldx % 8 ==
+ * x 4-byte and w8 16-byte aligned.  The weights stream once per 64 rows of M, or (x 16-byte
+ * aligned, ldx % 8 == 0, more than 16 rows, K <= 16384) once per up to 256 (the tile kernels).  With x 16-byte aligned and ldx % 8 ==
  * 0, up to 16 rows over 1024-4096 columns (up to 4 rows over at most 4096 columns) run without a K split (faster for
  * the decode GEMVs; the workspace is then unused). */
 int dsv41_fp8_gemm(const void* x, long ldx, const void* w8, const void* s8, int M, int N, int K, int Kc,

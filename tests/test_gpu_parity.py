@@ -954,6 +954,48 @@ def test_fp8_gemm(M, N, K, gc):
         assert (np.abs(got_u - want) <= 1e-5 * mag + 1e-30).all()
 
 
+@pytest.mark.parametrize("M,N,K,gc", [(17, 1280, 5120, 0), (24, 512, 5120, 0), (33, 200, 640, 0), (64, 100, 192, 0),
+                                      (65, 4096, 1280, 0), (100, 4096, 1280, 0), (130, 1024, 512, 128),
+                                      (129, 192, 320, 64), (257, 515, 1280, 0), (300, 2048, 1024, 256),
+                                      (1025, 512, 5120, 0), (2048, 8192, 1024, 0), (2100, 5120, 1024, 0),
+                                      (40, 96, 16384, 0), (20, 64, 16448, 0)])
+def test_fp8_gemm_many_rows(M, N, K, gc):
+    """The tile kernels (more than 16 rows) over their shapes, with and without K slices, row and column remainders and
+    block-diagonal groups, against float64 products of the dequantised weights; the last K runs the streaming kernel.
+    Bounds: fp32 chains of the streaming kernel's K slices, 1e-5 of the magnitudes (as the other kernels), the bf16 result one rounding
+    (half of the last of its 8 bits: at most 2^-8 of the value) and the 256-row shapes' longer chains (K products: sqrt(K) 2^-24 each way, under 1e-5) on top."""
+    from dsv41_amd.w8 import W8, fp8_gemm_tc
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    b = torch.randint(0, 256, (N, K), generator=g, device=DEV, dtype=torch.uint8)
+    b[(b & 0x7F) == 0x7F] = 0x01
+    s8 = torch.randint(100, 140, ((N + 31) // 32, K // 32), generator=g, device=DEV, dtype=torch.uint8)
+    w = W8(b, s8)
+    G = N // gc if gc else 1
+    x = torch.randn(M * G, K, generator=g, device=DEV).to(torch.bfloat16)
+    print(f"[fp8_gemm tiles] M {M} N {N} K {K} group_cols {gc}", flush=True)
+    got32 = fp8_gemm_tc(x, w.w8, w.s8, gc, out_dtype=torch.float32).double()
+    got16 = fp8_gemm_tc(x, w.w8, w.s8, gc).double()
+    wd = w.bf16().double()  # (exact: e4m3 values times powers of two within bf16's range)
+    prod = lambda x, w: (x @ w.t() if not gc else  # noqa: E731
+                         torch.cat([x[i::G] @ w[i * gc:(i + 1) * gc].t() for i in range(G)], 1))
+    want, mag = prod(x.double(), wd), prod(x.double().abs(), wd.abs())
+    assert bool(((got32 - want).abs() <= 1e-5 * mag + 1e-30).all()), float(((got32 - want).abs() / mag).max())
+    assert bool(((got16 - want).abs() <= 2 ** -8 * want.abs() * 1.01 + 1e-5 * mag + 1e-30).all())
+    if N <= 512 and not gc:  # narrow weights: the streaming kernel's bits (reached with x rows it cannot tile)
+        out = torch.empty(M, N, device=DEV, dtype=torch.bfloat16)
+        xs = torch.zeros(M, K + 2, device=DEV, dtype=torch.bfloat16)
+        xs[:, :K] = x
+        from dsv41_amd._lib import call, lib, ptr, stream
+        n = lib().dsv41_fp8_gemm_workspace_bytes(M, N, K)
+        ws = torch.zeros(n, dtype=torch.uint8, device=DEV)
+        call("dsv41_fp8_gemm", ptr(xs), K + 2, ptr(w.w8), ptr(w.s8), M, N, K, K // 32, 0, ptr(out), N, None, ptr(ws), n,
+             stream(x.device))
+        assert torch.equal(out.double(), got16)
+    xu = torch.empty(M * G * K + 2, device=DEV, dtype=torch.bfloat16)  # x only 4-byte aligned
+    xu[2:] = x.view(-1)
+    assert torch.equal(fp8_gemm_tc(xu[2:].view(M * G, K), w.w8, w.s8, gc).double(), got16)
+
+
 @pytest.mark.parametrize("mode,N,K", [(1, 1024, 1280), (2, 512, 8192), (1, 4096, 16384), (2, 300, 128), (1, 5120, 2048)])
 def test_fp8_gemv_m1_pre(mode, N, K):
     """fp8_gemv_m1_pre (dsv41/cukern.py:137-158): its prologue (norm_quant, dsv41/fused2.py:251-272; mode 2 the

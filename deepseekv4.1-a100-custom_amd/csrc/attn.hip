@@ -6,227 +6,15 @@
 //   dsv41_sattn2        fused2.sattn2                                    (SWA ring with position validity, then
 //                                                                         compressed rows by index; inverse rope)
 //
-// Work decomposition (gfx950, wave64): a workgroup of 4 waves owns one query row, 64 heads (wave w: heads
-// 16w..16w+15) and a contiguous chunk of that row's key list ("split").  Key rows are gathered 32 at a time into
-// LDS with 16-byte loads (invalid rows are zero-filled), shared by the 4 waves.  Per wave and tile:
-//   S^T[32 rows x 16 heads] = K * Q^T  -- 16x16x32 bf16 MFMA, A = K from LDS, B = Q held in VGPRs for the whole loop
-//   online softmax per head (fp32; max/sum across the 4 lane groups by shuffles)
-//   O[16 heads x DV] += P * V          -- the S^T accumulator of a lane already is the P operand (head = lane & 15,
-//                                         8 key rows), so P never leaves registers; V is read from the same LDS tile.
-// Several splits per row write fp32 partials (m, l, acc); a combine kernel merges them with the sink and applies
-// the inverse rope (dsv41/fused2.py:381-403).  A single split writes the final bf16 output directly.
+// Three kernels (gfx950, wave64), all on bf16 MFMA with fp32 softmax and accumulation: the 32-head and the 16-head
+// decode kernel for few query rows (key lists split over many workgroups, partials merged in the launch) and the
+// 64-head kernel for many rows (prefill chunks, serving batches; key splits merged by the combine kernel).
 #include <mutex>
 #include <type_traits>
 
 #include "attn_core.h"
 
 namespace {
-
-
-
-template <int DQK, int DV>
-__global__ void __launch_bounds__(256) attn_split_kernel(const AttnArgs a) {
-  constexpr int KS = DQK / 32;   // MFMA k-steps over the QK width
-  constexpr int CT = DV / 16;    // 16-wide output column tiles
-  constexpr int RSTR = DQK + 8;  // LDS row stride in elements (16 B pad)
-  constexpr int U = DQK / 8;     // 16-byte units per row
-  __shared__ __align__(16) uint16_t ktile[32 * RSTR];
-  __shared__ const uint16_t* rptr[32];
-
-  const int sp = blockIdx.x, hb = blockIdx.y, r = blockIdx.z;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int l16 = lane & 15, g = lane >> 4;
-  const int h0 = hb * 64 + wave * 16;
-  const int H = a.H;
-
-  uint4 qf[KS];
-  {
-    const int h = h0 + l16;
-    const uint16_t* qrow = a.q + (long)r * a.q_rstride + (long)h * DQK;
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
-      qf[ks] = h < H ? *(const uint4*)(qrow + ks * 32 + g * 8) : make_uint4(0, 0, 0, 0);
-  }
-
-  long slot, pos = 0, pmax = 0, plim = 0;
-  const int W = a.n1;
-  if (a.mode == 1) {
-    slot = a.seq[r];
-    pos = a.pos[r];
-    pmax = a.pmax[r];
-    plim = a.plim ? a.plim[r] : pos;
-  } else {
-    slot = r / a.rows_per_slot;
-  }
-  const uint16_t* base1 = a.kv1 + slot * a.kv1_sstride;
-  const uint16_t* base2 = a.kv2 ? a.kv2 + slot * a.kv2_sstride : nullptr;
-  const int* irow = a.t > 0 ? a.idx + (long)r * a.idx_rstride : nullptr;
-
-  float m_run = -1e30f, l_run = 0.0f;
-  f32x4_t o[CT];
-#pragma unroll
-  for (int c = 0; c < CT; ++c) o[c] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-
-  const int j0 = sp * a.chunk;
-  const int j1 = min(a.L, j0 + a.chunk);
-  for (int jt = j0; jt < j1; jt += 32) {
-    if (tid < 32) {
-      const int j = jt + tid;
-      const uint16_t* p = nullptr;
-      if (j < j1) {
-        if (a.mode == 1 && j < W) {
-          int m = (int)(pmax - j) % W;  // positions fit in 31 bits
-          m = m < 0 ? m + W : m;
-          const long held = pmax - m;
-          if (held >= 0 && held <= plim && pos - held < W) p = base1 + (long)j * DQK;
-        } else {
-          const int ix = irow[a.mode == 1 ? j - W : j];
-          if (a.mode == 1) {
-            if (ix >= 0 && ix < a.n2) p = base2 + (long)ix * DQK;
-          } else if (ix >= 0 && ix < a.n1 + a.n2) {
-            p = ix < a.n1 ? base1 + (long)ix * DQK : base2 + (long)(ix - a.n1) * DQK;
-          }
-        }
-      }
-      rptr[tid] = p;
-    }
-    __syncthreads();
-    for (int e = tid; e < 32 * U; e += 256) {
-      const int row = e / U, c = e - row * U;
-      const uint16_t* p = rptr[row];
-      const uint4 v = p ? *(const uint4*)(p + c * 8) : make_uint4(0, 0, 0, 0);
-      *(uint4*)(ktile + row * RSTR + c * 8) = v;
-    }
-    __syncthreads();
-
-    f32x4_t s[2];
-#pragma unroll
-    for (int rt = 0; rt < 2; ++rt) {
-      s[rt] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-      const uint16_t* krow = ktile + (rt * 16 + l16) * RSTR + g * 8;
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) s[rt] = mfma_bf16_16x16x32(*(const uint4*)(krow + ks * 32), qf[ks], s[rt]);
-    }
-    // s[rt][i] = score of key row rt*16 + 4g + i for head h0 + l16
-    float p[8];
-    float tmax = -1e30f;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int row = (e >> 2) * 16 + 4 * g + (e & 3);
-      const float x = rptr[row] ? s[e >> 2][e & 3] * a.scale : -1e30f;
-      p[e] = x;
-      tmax = fmaxf(tmax, x);
-    }
-    tmax = row_max4(tmax);
-    const float m_new = fmaxf(m_run, tmax);
-    const float alpha = exp2f((m_run - m_new) * kLog2e);
-    float psum = 0.0f;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int row = (e >> 2) * 16 + 4 * g + (e & 3);
-      p[e] = rptr[row] ? exp2f((p[e] - m_new) * kLog2e) : 0.0f;
-      psum += p[e];
-    }
-    psum = row_sum4(psum);
-    l_run = alpha * l_run + psum;
-    m_run = m_new;
-
-    float al[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) al[i] = __shfl(alpha, 4 * g + i, 64);
-    const uint4 pa = make_uint4(pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3]), pack_bf16x2(p[4], p[5]),
-                                pack_bf16x2(p[6], p[7]));
-    const uint16_t* vrow[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) vrow[e] = ktile + ((e >> 2) * 16 + 4 * g + (e & 3)) * RSTR + l16;
-#pragma unroll
-    for (int ct = 0; ct < CT; ++ct) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) o[ct][i] *= al[i];
-      const uint4 vb = make_uint4((uint32_t)vrow[0][ct * 16] | ((uint32_t)vrow[1][ct * 16] << 16),
-                                  (uint32_t)vrow[2][ct * 16] | ((uint32_t)vrow[3][ct * 16] << 16),
-                                  (uint32_t)vrow[4][ct * 16] | ((uint32_t)vrow[5][ct * 16] << 16),
-                                  (uint32_t)vrow[6][ct * 16] | ((uint32_t)vrow[7][ct * 16] << 16));
-      o[ct] = mfma_bf16_16x16x32(pa, vb, o[ct]);
-    }
-    __syncthreads();
-  }
-
-  if (a.nsplit == 1) {
-    const int hl = h0 + l16;
-    const float den = l_run + exp2f(((hl < H ? a.sink[hl] : 0.0f) - m_run) * kLog2e);
-    float inv[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) inv[i] = 1.0f / __shfl(den, 4 * g + i, 64);
-    long pr = pos < 0 ? 0 : pos;
-#pragma unroll
-    for (int ct = 0; ct < CT; ++ct) {
-      const int c = ct * 16 + l16;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        float v = round_bf16(o[ct][i] * inv[i]);
-        const float partner = dpp_mov<0xB1>(v);  // lane ^ 1
-        if (a.rd > 0 && c >= DV - a.rd) {
-          const int jj = (c - (DV - a.rd)) >> 1;
-          const float cs = a.cos_t[pr * (a.rd / 2) + jj];
-          const float sn = -a.sin_t[pr * (a.rd / 2) + jj];
-          v = (c & 1) ? (partner * sn + v * cs) : (v * cs - partner * sn);
-        }
-        const int h = h0 + 4 * g + i;
-        if (h < H) a.out[(long)r * a.out_rstride + (long)h * DV + c] = f2bf(v);
-      }
-    }
-  } else {
-    const int hl = h0 + l16;
-    if (g == 0 && hl < H) {
-      const long pi = ((long)r * H + hl) * a.nsplit + sp;
-      a.pm[pi] = m_run;
-      a.pl[pi] = l_run;
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int h = h0 + 4 * g + i;
-      if (h >= H) continue;
-      float* dst = a.pacc + (((long)r * H + h) * a.nsplit + sp) * DV;
-#pragma unroll
-      for (int ct = 0; ct < CT; ++ct) dst[ct * 16 + l16] = o[ct][i];
-    }
-  }
-}
-
-// Merge the splits of one (row, head): LSE combine + sink, bf16 round, inverse rope on the last rd columns.
-template <int DV>
-__global__ void __launch_bounds__(256) attn_combine_kernel(const AttnArgs a) {
-  const int h = blockIdx.x, r = blockIdx.y;
-  const int H = a.H, ns = a.nsplit;
-  const long base = ((long)r * H + h) * ns;
-  float mx = -1e30f;
-  for (int s = 0; s < ns; ++s) mx = fmaxf(mx, a.pm[base + s]);
-  float den = exp2f((a.sink[h] - mx) * kLog2e);
-  for (int s = 0; s < ns; ++s) den += a.pl[base + s] * exp2f((a.pm[base + s] - mx) * kLog2e);
-  const long pr = (a.mode == 1 && a.pos) ? (a.pos[r] < 0 ? 0 : a.pos[r]) : 0;
-  for (int c = 2 * threadIdx.x; c < DV; c += 512) {
-    float n0 = 0.0f, n1 = 0.0f;
-    for (int s = 0; s < ns; ++s) {
-      const float w = exp2f((a.pm[base + s] - mx) * kLog2e);
-      const float2 v = *(const float2*)(a.pacc + (base + s) * DV + c);
-      n0 += v.x * w;
-      n1 += v.y * w;
-    }
-    float re = round_bf16(n0 / den), im = round_bf16(n1 / den);
-    if (a.rd > 0 && c >= DV - a.rd) {
-      const int jj = (c - (DV - a.rd)) >> 1;
-      const float cs = a.cos_t[pr * (a.rd / 2) + jj];
-      const float sn = -a.sin_t[pr * (a.rd / 2) + jj];
-      const float yr = re * cs - im * sn, yi = re * sn + im * cs;
-      re = yr;
-      im = yi;
-    }
-    uint16_t* dst = a.out + (long)r * a.out_rstride + (long)h * DV + c;
-    dst[0] = f2bf(re);
-    dst[1] = f2bf(im);
-  }
-}
 
 // ------------------------------------------------------------------------------------------------ decode kernel
 // Few query rows (decode): the key list of a row is split across many workgroups, so each workgroup owns only 16
@@ -1073,11 +861,14 @@ __global__ void __launch_bounds__(512) attn_decode32_kernel(const AttnArgs a) {
 //       tile's 32 keys, each transposed V fragment used for four head blocks; the V fragments were read into VGPRs
 //       in iteration t - 1), interleaved with the direct-to-LDS gathers of tile t + 2 (counted vmcnt waits), then
 //       the V fragments of tile t - 1.
+// ROPE (rows that carry their rope in the attended width, the reference geometry): the inverse rope of the result and
+// fp32 split partials, as such rows always had them.  Replaced a 4-wave kernel without this overlap: 32 rows x 640 keys
+// of 512, kernel and combine 41.9 -> 29.5 us.
 // Four tile buffers: tile t (QK), t - 1 (V read by the PV waves), t + 1 and t + 2 (in flight; tile t + 2 goes into
 // tile t - 2's buffer, whose last read ended before B0).  B0: tile t has landed; P / rescale of tile t - 2 and the
 // row pointers of tile t + 2 are visible.  Keep the PV waves free of register
 // spills: a scratch reload waits for every outstanding load (vmcnt(0)), the in-flight gathers included.
-template <int DQK, int DV>
+template <int DQK, int DV, bool ROPE>
 __global__ void __launch_bounds__(512) attn_prefill_ws_kernel(const AttnArgs a) {
   constexpr int KS = DQK / 32;  // 32-deep k steps of QK^T
   constexpr int CT = DV / 64;   // 16-column output tiles per PV wave (a quarter of DV)
@@ -1088,7 +879,9 @@ __global__ void __launch_bounds__(512) attn_prefill_ws_kernel(const AttnArgs a) 
   constexpr int kLd = TILE * U / 256;  // loads per PV-wave lane per tile
   static_assert(TILE * U % 256 == 0 && kLd < 16, "vmcnt immediate");
   static_assert(64 * DV * 4 <= NBUF * TILE_ELEMS * 2, "output staging fits the tile buffers");
-  constexpr float kRescale = 8.0f;
+  // scores above the reference maximum before it moves (log2): with ROPE none, so a row's largest probability stays an
+  // exact 1 as in a plain softmax (the lazy reference of the other rows: relative error 2.19e-3 against 2.04e-3)
+  constexpr float kRescale = ROPE ? 0.0f : 8.0f;
   __shared__ __align__(16) uint16_t ktile[NBUF * TILE_ELEMS];
   __shared__ const uint16_t* rptr[NBUF][TILE];  // row of each key (the zero row when invalid: no test per gather)
   __shared__ uint32_t rvalid[NBUF];            // bit j: key j of the tile is valid
@@ -1438,18 +1231,40 @@ __global__ void __launch_bounds__(512) attn_prefill_ws_kernel(const AttnArgs a) 
     if (h >= H) continue;
     const float f = hfac[hl];
     const float4 x0 = *(const float4*)(stg + hl * DV + c), x1 = *(const float4*)(stg + hl * DV + c + 4);
-    const uint4 v = make_uint4(pack_bf16x2(x0.x * f, x0.y * f), pack_bf16x2(x0.z * f, x0.w * f),
-                               pack_bf16x2(x1.x * f, x1.y * f), pack_bf16x2(x1.z * f, x1.w * f));
-    if (a.nsplit > 1)  // bf16 partial [R, H, nsplit, DV] (merged by attn_decode_combine_kernel)
-      *(uint4*)((uint16_t*)a.pacc + (((long)r * H + h) * a.nsplit + sp) * DV + c) = v;
-    else
-      *(uint4*)(a.out + (long)r * a.out_rstride + (long)h * DV + c) = v;
+    if constexpr (ROPE) {
+      float v[8] = {x0.x * f, x0.y * f, x0.z * f, x0.w * f, x1.x * f, x1.y * f, x1.z * f, x1.w * f};
+      if (a.nsplit > 1) {  // fp32 partial [R, H, nsplit, DV] (merged by attn_decode_combine_kernel)
+        float* dst = a.pacc + (((long)r * H + h) * a.nsplit + sp) * DV + c;
+        *(float4*)dst = make_float4(v[0], v[1], v[2], v[3]);
+        *(float4*)(dst + 4) = make_float4(v[4], v[5], v[6], v[7]);
+        continue;
+      }
+      const long pr = pos < 0 ? 0 : pos;  // the inverse rope, of the bf16 result
+#pragma unroll
+      for (int q = 0; q < 8; q += 2) {
+        if (c + q < DV - a.rd) continue;
+        const long j = pr * (a.rd / 2) + ((c + q - (DV - a.rd)) >> 1);
+        const float cs = a.cos_t[j], sn = -a.sin_t[j], re = round_bf16(v[q]), im = round_bf16(v[q + 1]);
+        v[q] = re * cs - im * sn;
+        v[q + 1] = re * sn + im * cs;
+      }
+      *(uint4*)(a.out + (long)r * a.out_rstride + (long)h * DV + c) =
+          make_uint4(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]),
+                     pack_bf16x2(v[6], v[7]));
+    } else {
+      const uint4 v = make_uint4(pack_bf16x2(x0.x * f, x0.y * f), pack_bf16x2(x0.z * f, x0.w * f),
+                                 pack_bf16x2(x1.x * f, x1.y * f), pack_bf16x2(x1.z * f, x1.w * f));
+      if (a.nsplit > 1)  // bf16 partial [R, H, nsplit, DV] (merged by attn_decode_combine_kernel)
+        *(uint4*)((uint16_t*)a.pacc + (((long)r * H + h) * a.nsplit + sp) * DV + c) = v;
+      else
+        *(uint4*)(a.out + (long)r * a.out_rstride + (long)h * DV + c) = v;
+    }
   }
 }
 
-// Merge bf16-normalised partials: out = sum_s w_s l_s o_s / (sum_s w_s l_s + exp(sink - M)), w_s = exp(m_s - M).
+// Merge normalised partials (bf16, or fp32 with F32): out = sum_s w_s l_s o_s / (sum_s w_s l_s + exp(sink - M)), w_s = exp(m_s - M).
 // One workgroup per (row, 4 heads); thread -> (head, 8 consecutive columns); all split loads are independent.
-template <int DV>
+template <int DV, bool F32>
 __global__ void __launch_bounds__(256) attn_decode_combine_kernel(const AttnArgs a) {
   constexpr int MAXS = 32;  // splits held in registers; more are merged in further rounds
   constexpr int B = 8;      // partial rows loaded per batch
@@ -1459,7 +1274,34 @@ __global__ void __launch_bounds__(256) attn_decode_combine_kernel(const AttnArgs
   if (h >= H) return;
   const long base = ((long)r * H + h) * ns;
   const long pr = (a.mode == 1 && a.pos) ? (a.pos[r] < 0 ? 0 : a.pos[r]) : 0;
-  const uint16_t* pb = (const uint16_t*)a.pacc;
+  struct Part {
+    uint4 a, b;  // 8 columns of a partial row: bf16 in a, fp32 in both
+  };
+  auto load = [&](long s, int c) {
+    Part p;
+    if constexpr (F32) {
+      const uint4* src = (const uint4*)(a.pacc + (base + s) * DV + c);
+      p.a = src[0];
+      p.b = src[1];
+    } else {
+      p.a = *(const uint4*)((const uint16_t*)a.pacc + (base + s) * DV + c);
+      p.b = make_uint4(0, 0, 0, 0);
+    }
+    return p;
+  };
+  auto add = [](float (&num)[8], float w, const Part& p) {
+    const uint32_t x[8] = {p.a.x, p.a.y, p.a.z, p.a.w, p.b.x, p.b.y, p.b.z, p.b.w};
+    if constexpr (F32) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) num[e] += w * __uint_as_float(x[e]);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        num[2 * e] += w * __uint_as_float(x[e] << 16);
+        num[2 * e + 1] += w * __uint_as_float(x[e] & 0xffff0000u);
+      }
+    }
+  };
   // the inverse rope's cos / sin of the 4 column pairs at c (the last rd columns), issued with the partials'
   // loads and unconditionally (the zero row when there is no rope): one round trip instead of one per pair
   auto rope_load = [&](int c, float (&rc)[4], float (&rs)[4]) {
@@ -1493,12 +1335,12 @@ __global__ void __launch_bounds__(256) attn_decode_combine_kernel(const AttnArgs
   if (ns <= B && DV == 512) {
     // one round trip: the splits' maxima, sums and partial rows are loaded together (none depends on another)
     const int c = (threadIdx.x & 63) * 8;
-    uint4 v[B];
+    Part v[B];
     float m[B], l[B];
 #pragma unroll
     for (int u = 0; u < B; ++u) {
       const int s = u < ns ? u : ns - 1;
-      v[u] = *(const uint4*)(pb + (base + s) * DV + c);
+      v[u] = load(s, c);
       m[u] = u < ns ? a.pm[base + s] : -1e30f;
       l[u] = a.pl[base + s];
     }
@@ -1513,12 +1355,7 @@ __global__ void __launch_bounds__(256) attn_decode_combine_kernel(const AttnArgs
     for (int u = 0; u < B; ++u) {
       const float wg = u < ns ? l[u] * exp2f((m[u] - mx) * kLog2e) : 0.0f;
       den += wg;
-      const uint32_t vv[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        num[2 * e] += wg * __uint_as_float(vv[e] << 16);
-        num[2 * e + 1] += wg * __uint_as_float(vv[e] & 0xffff0000u);
-      }
+      add(num, wg, v[u]);
     }
     finish(c, num, den, rc, rs);
     return;
@@ -1538,23 +1375,18 @@ __global__ void __launch_bounds__(256) attn_decode_combine_kernel(const AttnArgs
     float num[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     float den = sink_term;
     for (int s0 = 0; s0 < ns; s0 += B) {
-      uint4 v[B];
+      Part v[B];
       float wg[B];
 #pragma unroll
       for (int u = 0; u < B; ++u) {
         const int s = s0 + u < ns ? s0 + u : ns - 1;
-        v[u] = *(const uint4*)(pb + (base + s) * DV + c);
+        v[u] = load(s, c);
         wg[u] = s0 + u < ns ? a.pl[base + s] * exp2f((a.pm[base + s] - mx) * kLog2e) : 0.0f;
       }
 #pragma unroll
       for (int u = 0; u < B; ++u) {
         den += wg[u];
-        const uint32_t vv[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          num[2 * e] += wg[u] * __uint_as_float(vv[e] << 16);
-          num[2 * e + 1] += wg[u] * __uint_as_float(vv[e] & 0xffff0000u);
-        }
+        add(num, wg[u], v[u]);
       }
     }
     finish(c, num, den, rc, rs);
@@ -1587,27 +1419,23 @@ int launch_attn(AttnArgs& a, hipStream_t st) {
     attn_decode_kernel<DQK, DV><<<grid, 512, 0, st>>>(a);
     DSV41_CHECK_LAUNCH();
     if (a.nsplit > 1 && !a.arrive) {
-      attn_decode_combine_kernel<DV><<<dim3((a.H + 3) / 4, a.R), 256, 0, st>>>(a);
+      attn_decode_combine_kernel<DV, false><<<dim3((a.H + 3) / 4, a.R), 256, 0, st>>>(a);
       DSV41_CHECK_LAUNCH();
     }
     return 0;
   }
-  dim3 grid(a.nsplit, (a.H + 63) / 64, a.R);
-  if (a.rd == 0) {  // (rows padded to a multiple of 8: contiguous row ranges per XCD)
-    attn_prefill_ws_kernel<DQK, DV><<<dim3(a.nsplit, grid.y, (a.R + kXcds - 1) / kXcds * kXcds), 512, 0, st>>>(a);
+  // (rows padded to a multiple of 8: contiguous row ranges per XCD)
+  const dim3 grid(a.nsplit, (a.H + 63) / 64, (a.R + kXcds - 1) / kXcds * kXcds), cgrid((a.H + 3) / 4, a.R);
+  if (a.rd > 0) {
+    attn_prefill_ws_kernel<DQK, DV, true><<<grid, 512, 0, st>>>(a);
     DSV41_CHECK_LAUNCH();
-    if (a.nsplit > 1) {  // bf16 partials merged with the sink
-      attn_decode_combine_kernel<DV><<<dim3((a.H + 3) / 4, a.R), 256, 0, st>>>(a);
-      DSV41_CHECK_LAUNCH();
-    }
-    return 0;
+    if (a.nsplit > 1) attn_decode_combine_kernel<DV, true><<<cgrid, 256, 0, st>>>(a);
+  } else {
+    attn_prefill_ws_kernel<DQK, DV, false><<<grid, 512, 0, st>>>(a);
+    DSV41_CHECK_LAUNCH();
+    if (a.nsplit > 1) attn_decode_combine_kernel<DV, false><<<cgrid, 256, 0, st>>>(a);
   }
-  attn_split_kernel<DQK, DV><<<grid, 256, 0, st>>>(a);
   DSV41_CHECK_LAUNCH();
-  if (a.nsplit > 1) {
-    attn_combine_kernel<DV><<<dim3(a.H, a.R), 256, 0, st>>>(a);
-    DSV41_CHECK_LAUNCH();
-  }
   return 0;
 }
 
@@ -1642,7 +1470,7 @@ constexpr int kDecWG = DSV41_DEC_WG;
   // decode-kernel workgroups the split plan aims at
 
 // Split plan.  Decode kernel: <= 192 workgroups over (rows x 16-head groups x splits), >= 2 tiles of 64 keys per
-// split.  64-head kernel: splits up to one workgroup per CU when rows are few, >= 2 tiles of 32 keys per split.
+// split.  64-head kernel: up to 8 splits, one workgroup per CU, when rows are few, >= 3 tiles of 32 keys per split.
 // The 32-head decode kernel's plan (automatic split count only, DV a multiple of 128): splits of 128 keys (64 when that leaves fewer than
 // 96 workgroups), 8 to 64 of them, every workgroup resident at once (one per CU; the head groups of a (row, split) on one
 // XCD).  DSV41_ATTN_DEC32=0 selects the 16-head kernel instead.  Returns false when it does not apply.
@@ -1684,7 +1512,14 @@ void plan(int R, int H, int L, int want, int dv, int* nsplit, int* chunk) {
     const long cus = (long)cus_per_xcd() * kXcds > 0 ? (long)cus_per_xcd() * kXcds : 256;
     const long target = wgs >= cus ? 1 : cus / wgs;
     per = (int)((tiles + target - 1) / target);
-    if (per < 2 && target > 1) per = 2;
+    // up to 8 splits (the combine then loads a row's partials in one round trip: 16 rows x 2176 keys of 576, 8 splits
+    // 27.4 us, 14 30.4 us) of at least 3 tiles (16 rows x 640 keys of 512: 7 splits 26.8 us, 10 29.7 us), and two of
+    // at least 12 (128 rows x 640 keys: one 38.6 us, two 43.7 us)
+    if (target > 1) {
+      per = per < 3 ? 3 : per;
+      per = per < (tiles + 7) / 8 ? (tiles + 7) / 8 : per;
+      if (target == 2 && per < 12) per = tiles;
+    }
   }
   if (per < 1) per = 1;
   if (per > tiles) per = tiles;

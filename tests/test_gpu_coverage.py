@@ -56,9 +56,10 @@ def _rope_tables(rd, n):
 
 
 # ------------------------------------------------------------------------------------------ many-row attention
-@pytest.mark.parametrize("dqk,R,k,n", [(576, 32, 2048, 6000), (576, 48, 300, 250), (512, 24, 512, 9000)])
-def test_sattn2_many_rows_unit_scale(dqk, R, k, n):
-    """The 64-head kernel at values of unit size against a float64 softmax, three launches bit-equal: gathers still in
+@pytest.mark.parametrize("dqk,R,k,n,nsplit", [(576, 32, 2048, 6000, 0), (576, 48, 300, 250, 0), (512, 24, 512, 9000, 0),
+                                              (512, 16, 512, 700, 1), (512, 40, 130, 4000, 3), (512, 300, 100, 99, 0)])
+def test_sattn2_many_rows_unit_scale(dqk, R, k, n, nsplit):
+    """The 64-head kernel, with (512) and without (576) the inverse rope of the result, at values of unit size against a float64 softmax, three launches bit-equal: gathers still in
     flight when the output is staged would show in single elements.  Rows end in empty entries as short contexts do.
     Bound per output row: bf16 probabilities, partials and result round by at most 2^-8, in the 2-norm by under 2^-8.5
     each (independent): sqrt(3) 2^-8.5 < 2^-7."""
@@ -77,8 +78,8 @@ def test_sattn2_many_rows_unit_scale(dqk, R, k, n):
     seq = torch.arange(R, device=DEV)
     cos, sin = (x.to(DEV) for x in _rope_tables(64, 8192))
     rd = 64 if dqk == 512 else 0
-    got = [dsv41_amd.sattn2(q, ring, ckv, idx.unsqueeze(1), pos, sink, cos, sin, rd, dqk ** -0.5, seq, pos, d_v=dv)
-           for _ in range(3)]
+    got = [dsv41_amd.sattn2(q, ring, ckv, idx.unsqueeze(1), pos, sink, cos, sin, rd, dqk ** -0.5, seq, pos, d_v=dv,
+                            nsplit=nsplit) for _ in range(3)]
     assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
     for r in range(R):
         sel = idx[r][idx[r] >= 0].long()

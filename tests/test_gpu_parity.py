@@ -95,6 +95,63 @@ def _fp8_close(got, want, tag):
         assert rel.max() <= 0.34, (tag, rel.max())
 
 
+@pytest.mark.parametrize("group,mode", [(32, 0), (16, 0), (32, 1), (16, 1), (32, 2), (16, 2)])
+def test_row_operations_aligned_and_not(group, mode):
+    """Fake quantisation and rope of 16-byte aligned rows (flat, 16 bytes a lane) against the same values at an odd
+    alignment (row kernels), bit for bit: zeros of both signs, subnormal results, infinities, NaN, a last workgroup
+    that is not full."""
+    import dsv41_amd
+    g = torch.Generator(device=DEV).manual_seed(9)
+
+    def wide(*s):
+        v = torch.randn(*s, generator=g, device=DEV) * torch.exp2(torch.randint(-30, 12, s, generator=g, device=DEV).float())
+        v[torch.rand(s, generator=g, device=DEV) < 0.05] = -0.0
+        return v.to(torch.bfloat16)
+
+    def odd(x):
+        y = torch.empty(x.numel() + 2, dtype=x.dtype, device=DEV)[2:].view(x.shape)
+        return y.copy_(x)
+
+    def same(a, b):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+
+    for D in (group, 96, 576, 1024):
+        x = wide(37, D)
+        x[3, 5], x[4, 7], x[5] = float("inf"), float("nan"), 0.0
+        same(dsv41_amd.fake_quant(x, group, mode), dsv41_amd.fake_quant(odd(x), group, mode))
+    cos, sin = torch.rand(64, 32, generator=g, device=DEV), torch.rand(64, 32, generator=g, device=DEV)
+    for shape in ((1, 9, 64, 512), (2, 5, 3, 72), (3, 7, 576)):
+        x = wide(*shape)
+        y = odd(x)
+        for inverse in (False, True):
+            dsv41_amd.rope_(x, 64, cos, sin, 5, inverse, 4)
+            dsv41_amd.rope_(y, 64, cos, sin, 5, inverse, 4)
+            same(x, y)
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 1003])
+def test_index_key_conversion_aligned_and_not(n):
+    """The converters' 16-byte form against the general one (tables at an odd alignment), bit for bit: row remainders,
+    values far below the row's maximum (subnormal codes, zeros of both signs), every byte code."""
+    from dsv41_amd._lib import call, ptr, stream
+    g = torch.Generator(device=DEV).manual_seed(n)
+    k = (torch.randn(n, 128, generator=g, device=DEV) *
+         torch.exp2(torch.randint(-24, 4, (n, 128), generator=g, device=DEV).float())).to(torch.bfloat16)
+    k[0, :7] = -0.0
+    st = stream(k.device)
+    res = []
+    for off in (0, 2):
+        src = torch.empty(n * 128 + off, dtype=torch.bfloat16, device=DEV)[off:].view(n, 128).copy_(k)
+        k8 = torch.zeros(n, 128, dtype=torch.uint8, device=DEV)
+        ks = torch.zeros(n, device=DEV)
+        call("dsv41_index_keys_encode", ptr(src), n, ptr(k8), ptr(ks), st)
+        codes = torch.arange(256, device=DEV, dtype=torch.uint8).repeat((n + 1) // 2)[:n * 128].view(n, 128).contiguous()
+        out = torch.zeros(n * 128 + off, dtype=torch.bfloat16, device=DEV)[off:].view(n, 128)
+        call("dsv41_index_keys_decode", ptr(codes), ptr(ks), n, ptr(out), st)
+        res.append((k8, ks, out.clone().view(torch.int16)))
+    assert all(torch.equal(a, b) for a, b in zip(*res))
+
+
 @pytest.mark.parametrize("D", [512, 576])
 def test_kv_write(D):
     import dsv41_amd

@@ -9,7 +9,7 @@ from __future__ import annotations
 
 import torch
 
-from ._lib import as_i64, call, ptr, require_gpu, stream
+from ._lib import as_bf16, as_i64, as_rows, call, ptr, require_gpu, stream
 
 
 _WIDX = {}  # window index tensors by shape: functions of (window, bsz, seqlen, start_pos or history length) only
@@ -59,7 +59,7 @@ def window_kv(kv_raw: torch.Tensor, norm_w: torch.Tensor, eps: float, cos: torch
     dev = require_gpu(kv_raw, ring, cos, sin)
     W = ring.shape[1]
     x = kv_raw.reshape(b * s, d).contiguous()
-    w = norm_w.to(torch.bfloat16).contiguous()
+    w = as_bf16(norm_w)
     st = stream(dev)
     if s == 1 and start_pos > 0:
         call("dsv41_kv_write", ptr(x), d, ptr(w), ptr(cos), ptr(sin), None, None, start_pos, 0, 1, ptr(ring),
@@ -114,7 +114,8 @@ def write_index_k(cache: torch.Tensor, k_raw: torch.Tensor, norm_w: torch.Tensor
             raise RuntimeError(f"write_index_k: rows {start_pos // ratio}+{n} x {b} do not fit {tuple(tab.shape)}")
     first = start_pos - (start_pos % ratio)
     x = k_raw.reshape(b * n, D).contiguous()
-    call("dsv41_append_rows", ptr(x), D, ptr(norm_w.to(torch.bfloat16).contiguous()), float(eps), ptr(cos), ptr(sin),
+    w = as_bf16(norm_w)
+    call("dsv41_append_rows", ptr(x), D, ptr(w), float(eps), ptr(cos), ptr(sin),
          rd, None, first, ratio, 0, None, n, None, start_pos // ratio, ptr(cache), cache.stride(0), 1, 32,
          ptr(k8) if k8 is not None else None, k8.stride(0) if k8 is not None else 0,
          ptr(k_scale) if k_scale is not None else None, k_scale.stride(0) if k_scale is not None else 0, b * n, D,
@@ -126,13 +127,13 @@ def append_compressed_decode(cache: torch.Tensor, latent: torch.Tensor, pos: tor
     """Decode compressed append (dsv41/decode.py:157-162): rope_dev_(latent, add = 1 - ratio) -> fq4(16, e4m3) ->
     cache[seq, row] (row = compress_len - 1 when the group closed, else the caller's spare row)."""
     D = latent.shape[-1]
-    x = latent.reshape(-1, D).contiguous()
+    x = as_rows(latent, D)
     B = x.shape[0]
     dev = require_gpu(x, cache)
+    pos, seq, row = as_i64(pos, dev), as_i64(seq, dev), as_i64(row, dev)
     assert cache.stride(2) == 1 and cache.stride(1) == D
-    call("dsv41_append_rows", ptr(x), D, None, 0.0, ptr(cos), ptr(sin), rd, ptr(as_i64(pos.reshape(-1), dev)), 0, 0,
-         1 - ratio, ptr(as_i64(seq.reshape(-1), dev)), 1, ptr(as_i64(row.reshape(-1), dev)), 0, ptr(cache),
-         cache.stride(0), 2, 16, None, 0, None, 0, B, D, stream(dev))
+    call("dsv41_append_rows", ptr(x), D, None, 0.0, ptr(cos), ptr(sin), rd, ptr(pos), 0, 0,
+         1 - ratio, ptr(seq), 1, ptr(row), 0, ptr(cache), cache.stride(0), 2, 16, None, 0, None, 0, B, D, stream(dev))
 
 
 def append_index_k_decode(cache: torch.Tensor, k_raw: torch.Tensor, norm_w: torch.Tensor, eps: float,
@@ -142,14 +143,14 @@ def append_index_k_decode(cache: torch.Tensor, k_raw: torch.Tensor, norm_w: torc
     """Decode index-key append (dsv41/decode.py:270-282): rmsnorm -> rope_dev_(add = 1 - ratio) -> fq4(32) ->
     cache[seq, row] (bf16, the reference storage; may be None) and/or the e4m3 copy k8[seq, row] + k_scale."""
     D = k_raw.shape[-1]
-    x = k_raw.reshape(-1, D).contiguous()
+    x = as_rows(k_raw, D)
     B = x.shape[0]
     dev = require_gpu(x, cache, k8)
+    pos, seq, row, w = as_i64(pos, dev), as_i64(seq, dev), as_i64(row, dev), as_bf16(norm_w)
     if cache is None and k8 is None:
         raise RuntimeError("append_index_k_decode: no destination table")
-    call("dsv41_append_rows", ptr(x), D, ptr(norm_w.to(torch.bfloat16).contiguous()), float(eps), ptr(cos), ptr(sin),
-         rd, ptr(as_i64(pos.reshape(-1), dev)), 0, 0, 1 - ratio, ptr(as_i64(seq.reshape(-1), dev)), 1,
-         ptr(as_i64(row.reshape(-1), dev)), 0, ptr(cache), cache.stride(0) if cache is not None else 0, 1, 32,
+    call("dsv41_append_rows", ptr(x), D, ptr(w), float(eps), ptr(cos), ptr(sin),
+         rd, ptr(pos), 0, 0, 1 - ratio, ptr(seq), 1, ptr(row), 0, ptr(cache), cache.stride(0) if cache is not None else 0, 1, 32,
          ptr(k8) if k8 is not None else None, k8.stride(0) if k8 is not None else 0,
          ptr(k_scale) if k_scale is not None else None, k_scale.stride(0) if k_scale is not None else 0, B, D,
          stream(dev))
@@ -157,7 +158,7 @@ def append_index_k_decode(cache: torch.Tensor, k_raw: torch.Tensor, norm_w: torc
 
 def _nw(nw_tab, dev):
     """The no-write row table as contiguous int64 on the launch device (None stays None)."""
-    return None if nw_tab is None else as_i64(nw_tab.reshape(-1), dev)
+    return None if nw_tab is None else as_i64(nw_tab, dev)
 
 
 def decode_appends(kv_raw, kv_norm, ring, latent, ckv, k_raw, k_norm, kbf, k8, k_scale, pos, seq, ratio: int,
@@ -172,23 +173,26 @@ def decode_appends(kv_raw, kv_norm, ring, latent, ckv, k_raw, k_norm, kbf, k8, k
     wf [B, 64] of the e4m3 score path."""
     dev = require_gpu(kv_raw, ring, latent, ckv, k_raw, kbf, k8)
     Dw = ring.shape[-1]
-    x = kv_raw.reshape(-1, Dw).contiguous()
+    x = as_rows(kv_raw, Dw)
     B = x.shape[0]
+    # (converted operands are held here until the launch: a dropped one's memory could be reused before it)
+    pos, seq, nw = as_i64(pos, dev), as_i64(seq, dev), _nw(nw_tab, dev)
+    kv_norm, k_norm = as_bf16(kv_norm), as_bf16(k_norm) if k_norm is not None else None
+    if q_idx is not None:
+        q_idx, w_idx = q_idx.contiguous(), as_bf16(w_idx)
     assert ring.stride(2) == 1 and ring.stride(1) == Dw
     lat = latent.reshape(B, -1).contiguous() if latent is not None else None
     kr = k_raw.reshape(B, -1).contiguous() if k_raw is not None else None
     tab = k8 if k8 is not None else kbf
     Dk = tab.shape[-1] if tab is not None else 128
     kcap = tab.shape[1] if tab is not None else 1
-    call("dsv41_decode_appends", ptr(x), ptr(kv_norm.to(torch.bfloat16).contiguous()), ptr(ring), ring.stride(0),
+    call("dsv41_decode_appends", ptr(x), ptr(kv_norm), ptr(ring), ring.stride(0),
          ring.shape[1], Dw, ptr(lat), ptr(ckv), ckv.stride(0) if ckv is not None else 0,
-         ckv.shape[1] if ckv is not None else 1, ptr(kr),
-         ptr(k_norm.to(torch.bfloat16).contiguous()) if k_norm is not None else None, ptr(kbf),
+         ckv.shape[1] if ckv is not None else 1, ptr(kr), ptr(k_norm), ptr(kbf),
          kbf.stride(0) if kbf is not None else 0, ptr(k8), k8.stride(0) if k8 is not None else 0, ptr(k_scale),
-         k_scale.stride(0) if k_scale is not None else 0, kcap, Dk, ptr(as_i64(pos.reshape(-1), dev)),
-         ptr(as_i64(seq.reshape(-1), dev)), ptr(_nw(nw_tab, dev)), int(ratio), ptr(cos), ptr(sin), int(rd), float(eps),
-         ptr(q_idx.contiguous()) if q_idx is not None else None,
-         ptr(w_idx.to(torch.bfloat16).contiguous()) if q_idx is not None else None,
+         k_scale.stride(0) if k_scale is not None else 0, kcap, Dk, ptr(pos), ptr(seq), ptr(nw),
+         int(ratio), ptr(cos), ptr(sin), int(rd), float(eps),
+         ptr(q_idx), ptr(w_idx) if q_idx is not None else None,
          q_idx.shape[-2] if q_idx is not None else 0, ptr(q8), ptr(wf), B, stream(dev))
 
 

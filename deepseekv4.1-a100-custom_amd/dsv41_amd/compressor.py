@@ -5,7 +5,7 @@ from __future__ import annotations
 
 import torch
 
-from ._lib import as_i64, call, ptr, require_gpu, stream
+from ._lib import as_bf16, as_f32, as_i64, call, ptr, require_gpu, stream
 
 RING = 8  # positions kept per sequence (Compressor.RING, dsv41/model.py:588)
 
@@ -27,9 +27,9 @@ def compress_pool(kv: torch.Tensor, score: torch.Tensor, start_pos: int, ratio: 
     first_end = start_pos + (ratio - 1 - start_pos % ratio)
     last = start_pos + s - 1
     n_groups = (last - first_end) // ratio + 1 if first_end <= last else 0
-    kvc = kv.float().contiguous()
-    scc = score.float().contiguous()
-    w = norm_w.to(torch.bfloat16).contiguous()
+    kvc = as_f32(kv)
+    scc = as_f32(score)
+    w = as_bf16(norm_w)
     out = torch.empty(b, n_groups, D, dtype=torch.bfloat16, device=dev)
     assert ring_kv.is_contiguous() and ring_score.is_contiguous() and ring_kv.shape == ring_score.shape
     for bi in range(b):
@@ -46,13 +46,14 @@ def compress_pool_decode(kv: torch.Tensor, score: torch.Tensor, pos: torch.Tenso
     at positions pos of sequences seq.  Returns (latent bf16 [B, 1, D], should bool [B]); updates the rings."""
     dev = require_gpu(kv, score, ring_kv, ring_score)
     D = kv.shape[-1]
-    kvc = kv.reshape(-1, D).float().contiguous()
-    scc = score.reshape(-1, D).float().contiguous()
+    kvc = as_f32(kv.reshape(-1, D))
+    scc = as_f32(score.reshape(-1, D))
+    pos, seq, w = as_i64(pos, dev), as_i64(seq, dev), as_bf16(norm_w)
     B = kvc.shape[0]
     latent = torch.empty(B, 1, D, dtype=torch.bfloat16, device=dev)
     should = torch.empty(B, dtype=torch.bool, device=dev)
     assert ring_kv.is_contiguous() and ring_score.is_contiguous()
     call("dsv41_compress_pool_decode", ptr(kvc), ptr(scc), D, ptr(ring_kv), ptr(ring_score), ring_kv.stride(0),
-         ring_kv.shape[1], ptr(as_i64(pos.reshape(-1), dev)), ptr(as_i64(seq.reshape(-1), dev)), B, D, int(ratio),
-         ptr(norm_w.to(torch.bfloat16).contiguous()), float(eps), ptr(latent), D, ptr(should), stream(dev))
+         ring_kv.shape[1], ptr(pos), ptr(seq), B, D, int(ratio),
+         ptr(w), float(eps), ptr(latent), D, ptr(should), stream(dev))
     return latent, should

@@ -70,8 +70,8 @@ class DecodeLayer:
                    k_norm=k_norm, kbf=self.kbf16, k8=self.k8, k_scale=self.ks, ratio=self.ratio, cos=self.cos,
                    sin=self.sin, rd=self.rd, eps=self.eps, q_idx=q_idx, w_idx=w_idx, nw_tab=self.nw_tab)
         self._prepared = None
-        return sel.select_with_appends(app, as_i64(pos.reshape(-1), dev), as_i64(seq.reshape(-1), dev),
-                                       as_i64(cl.reshape(-1), dev), cand)
+        return sel.select_with_appends(app, as_i64(pos, dev), as_i64(seq, dev),
+                                       as_i64(cl, dev), cand)
 
     def select(self, q_idx, w_idx, pos, seq, cl=None):
         """Indexer score over the e4m3 keys + top-k (dsv41/decode.py:284-294), histogram-assisted selection."""

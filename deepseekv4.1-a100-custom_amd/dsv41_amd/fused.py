@@ -4,7 +4,7 @@ from __future__ import annotations
 
 import torch
 
-from ._lib import as_i64, call, ptr, require_gpu, stream
+from ._lib import as_bf16, as_f32, as_i64, call, ptr, require_gpu, stream
 
 
 def fake_quant(x: torch.Tensor, group: int, mode: int) -> torch.Tensor:
@@ -39,7 +39,8 @@ def rmsnorm(x: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
     if D > 1024 and xc.data_ptr() % 16:  # long rows go through 16-byte loads
         xc = xc.clone()
     y = torch.empty_like(xc)
-    call("dsv41_rmsnorm", ptr(xc), ptr(w.to(torch.bfloat16).contiguous()), ptr(y), xc.numel() // D, D, float(eps),
+    wc = as_bf16(w)
+    call("dsv41_rmsnorm", ptr(xc), ptr(wc), ptr(y), xc.numel() // D, D, float(eps),
          stream(dev))
     return y
 
@@ -55,7 +56,7 @@ def norm_quant(x: torch.Tensor, w: torch.Tensor | None, eps: float) -> torch.Ten
     if xc.data_ptr() % 16:
         xc = xc.clone()
     y = torch.empty_like(xc)
-    wc = None if w is None else w.to(torch.bfloat16).contiguous()
+    wc = None if w is None else as_bf16(w)
     call("dsv41_norm_quant", ptr(xc), ptr(wc), float(eps), ptr(y), xc.numel() // D, D, stream(dev))
     return y
 
@@ -87,7 +88,7 @@ def rope_dev_(x: torch.Tensor, rd: int, cos: torch.Tensor, sin: torch.Tensor, po
     assert x.is_contiguous()
     dev = require_gpu(x, cos, sin)
     b, s, h, d = _rope_shape(x)
-    p = as_i64(pos.reshape(-1), dev)
+    p = as_i64(pos, dev)
     call("dsv41_rope", ptr(x), ptr(cos), ptr(sin), ptr(p), 0, int(add), int(pos_stride), b * s * h, h, s, d, rd,
          int(inverse), stream(dev))
     return x
@@ -119,7 +120,7 @@ def sparse_attn_decode2(q, kv1, kv2, attn_sink, topk_idxs, softmax_scale, nsplit
     k2 = kv2.contiguous() if kv2 is not None else None
     idx = topk_idxs.to(torch.int32).contiguous()
     t = idx.shape[-1]
-    sink = attn_sink.float().contiguous()
+    sink = as_f32(attn_sink)
     o = torch.empty_like(qc)
     ws, n = _workspace(dev, b, h, t, d, nsplit)
     call("dsv41_sparse_attn2", ptr(qc), ptr(k1), ptr(k2), ptr(sink), ptr(idx), ptr(o), b, h, d, k1.shape[1],

@@ -5,7 +5,7 @@ from __future__ import annotations
 import torch
 
 from . import _lib
-from ._lib import as_i64, attn_error_word, call, check_error_word, lib, ptr, require_gpu, stream
+from ._lib import as_bf16, as_f32, as_i64, as_rows, attn_error_word, call, check_error_word, lib, ptr, require_gpu, stream
 
 
 def kv_write(x: torch.Tensor, w: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, pos: torch.Tensor,
@@ -13,14 +13,15 @@ def kv_write(x: torch.Tensor, w: torch.Tensor, cos: torch.Tensor, sin: torch.Ten
     """dsv41/fused2.py:303-330: x bf16 [B, d]; pos, seq int64 [B]; cache [S, W, d] ring, written at
     [seq, pos % W] with rmsnorm -> rope -> fp8 fake quant."""
     dev = require_gpu(x, cache, cos, sin)
-    pos = as_i64(pos.reshape(-1), dev)
-    seq = as_i64(seq.reshape(-1), dev)
+    pos = as_i64(pos, dev)
+    seq = as_i64(seq, dev)
     d = x.shape[-1]
     win = cache.shape[1]
-    xc = x.reshape(-1, d).contiguous()
+    xc = as_rows(x, d)
+    wc = as_bf16(w)
     B = xc.shape[0]
     assert cache.stride(2) == 1 and cache.stride(1) == d
-    call("dsv41_kv_write", ptr(xc), d, ptr(w.to(torch.bfloat16).contiguous()), ptr(cos), ptr(sin), ptr(pos), ptr(seq),
+    call("dsv41_kv_write", ptr(xc), d, ptr(wc), ptr(cos), ptr(sin), ptr(pos), ptr(seq),
          0, 0, 1, ptr(cache), cache.stride(0), win, None, B, d, rd, float(eps), 0, stream(dev))
 
 
@@ -38,10 +39,10 @@ def sattn2(q, kv_win, kv_c, idx, pos, attn_sink, cos, sin, rd, softmax_scale, se
     qc = q.contiguous()
     win = kv_win.shape[1]
     assert kv_win.stride(2) == 1 and kv_win.stride(1) == d
-    pos = as_i64(pos.reshape(-1), dev)
-    seq = as_i64(seq.reshape(-1), dev)
-    pmax = as_i64(pmax.reshape(-1), dev)
-    plim = as_i64(plim.reshape(-1), dev) if plim is not None else None
+    pos = as_i64(pos, dev)
+    seq = as_i64(seq, dev)
+    pmax = as_i64(pmax, dev)
+    plim = as_i64(plim, dev) if plim is not None else None
     if kv_c is None or idx is None:
         kvc, c_stride, n_c, ix, t = None, 0, 0, None, 0
     else:
@@ -49,7 +50,7 @@ def sattn2(q, kv_win, kv_c, idx, pos, attn_sink, cos, sin, rd, softmax_scale, se
         kvc, c_stride, n_c = kv_c, kv_c.stride(0), kv_c.shape[1]
         ix = idx.to(torch.int32).reshape(b, -1).contiguous()
         t = ix.shape[-1]
-    sink = attn_sink.float().contiguous()
+    sink = as_f32(attn_sink)
     o = torch.empty(b, 1, h, dv, device=dev, dtype=q.dtype)
     nbytes = lib().dsv41_attn_workspace_bytes(b, h, win + t, dv, nsplit)
     if ws is None:  # the split-arrival counters at its start must be zero at first use; launches leave them ready

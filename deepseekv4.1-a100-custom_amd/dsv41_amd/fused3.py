@@ -5,7 +5,7 @@ from __future__ import annotations
 import torch
 
 from . import _lib
-from ._lib import as_i64, call, check_error_word, lib, ptr, require_gpu, stream
+from ._lib import as_bf16, as_f32, as_i64, as_rows, call, check_error_word, lib, ptr, require_gpu, stream
 
 
 def qprep(q: torch.Tensor, weights: torch.Tensor):
@@ -14,8 +14,9 @@ def qprep(q: torch.Tensor, weights: torch.Tensor):
     dev = q.device
     q8 = torch.empty(B, 64, 128, dtype=torch.uint8, device=dev)
     wf = torch.empty(B, 64, dtype=torch.float32, device=dev)
-    w = weights.reshape(B, H).float().contiguous()
-    call("dsv41_index_qprep", ptr(q.contiguous()), ptr(w), B, H, ptr(q8), ptr(wf), stream(dev))
+    qc = q.contiguous()
+    w = as_f32(weights.reshape(B, H))
+    call("dsv41_index_qprep", ptr(qc), ptr(w), B, H, ptr(q8), ptr(wf), stream(dev))
     return q8, wf
 
 
@@ -47,7 +48,7 @@ def _score(q, index_k, weights, seq, cl, k_scale, out, write_masked: bool, hist,
              cp, cs, stream(dev))
     else:
         qc = q.contiguous()
-        w = weights.reshape(B, H).float().contiguous()
+        w = as_f32(weights.reshape(B, H))
         call("dsv41_index_score", ptr(qc), H * D, ptr(w), H, B, H, D, 0, ptr(index_k), index_k.stride(0), None, 0,
              ptr(seq), 1, ptr(cl), 0, 1, n_pos, int(write_masked), ptr(out), out.stride(0), ptr(hist), cp, cs,
              stream(dev))
@@ -62,7 +63,7 @@ def index_score(q: torch.Tensor, index_k: torch.Tensor, weights: torch.Tensor, s
     B, _, H, D = q.shape
     dev = require_gpu(q, index_k, weights)
     out = torch.empty(B, index_k.shape[1], device=dev, dtype=torch.float32)
-    _score(q, index_k, weights, as_i64(seq.reshape(-1), dev), as_i64(cl.reshape(-1), dev), k_scale, out, True, None,
+    _score(q, index_k, weights, as_i64(seq, dev), as_i64(cl, dev), k_scale, out, True, None,
            cand=cand)
     return out
 
@@ -73,7 +74,7 @@ def topk_indices(score: torch.Tensor, k: int, cl: torch.Tensor) -> torch.Tensor:
     B, n = score.shape
     dev = require_gpu(score)
     assert score.stride(-1) == 1
-    cl = as_i64(cl.reshape(-1), dev)
+    cl = as_i64(cl, dev)
     out = torch.empty(B, k, device=dev, dtype=torch.int32)
     call("dsv41_topk_indices", ptr(score), score.stride(0), B, n, k, ptr(cl), 0, 1, 1, 0, ptr(out), k, stream(dev))
     return out.view(B, 1, k)
@@ -153,36 +154,36 @@ class DecodeSelector:
         dev = self.score.device
         ring, ckv, k8, ks, kbf = app["ring"], app.get("ckv"), app["k8"], app["k_scale"], app.get("kbf")
         Dw = ring.shape[-1]
-        x = app["kv_raw"].reshape(-1, Dw).contiguous()
+        x = as_rows(app["kv_raw"], Dw)
         B = x.shape[0]
         if B != self.rows or k8.shape[1] != self.n_pos or k8.shape[-1] != 128:
             raise RuntimeError(f"select_with_appends: built for {self.rows} x {self.n_pos}, got {B} x {k8.shape[1]}")
         lat = app["latent"].reshape(B, -1).contiguous() if app.get("latent") is not None else None
-        q_idx, w_idx = app["q_idx"], app["w_idx"]
+        # (converted operands are held here until the launch: a dropped one's memory could be reused before it)
+        q_idx, w_idx, k_raw = app["q_idx"].contiguous(), as_bf16(app["w_idx"]), app["k_raw"].reshape(B, -1).contiguous()
+        kv_norm, k_norm = as_bf16(app["kv_norm"]), as_bf16(app["k_norm"])
         HI = q_idx.shape[-2]
         assert ring.stride(2) == 1 and ring.stride(1) == Dw and ks.dtype == torch.float32
         nw = app.get("nw_tab")
-        nw = as_i64(nw.reshape(-1), dev) if nw is not None else None
+        nw = as_i64(nw, dev) if nw is not None else None
         if not self.one_launch:
             cp, cs = _cand_args(cand, self.rows, self.n_pos)
-            call("dsv41_decode_score", ptr(x), ptr(app["kv_norm"].to(torch.bfloat16).contiguous()), ptr(ring),
+            call("dsv41_decode_score", ptr(x), ptr(kv_norm), ptr(ring),
                  ring.stride(0), ring.shape[1], Dw, ptr(lat), ptr(ckv), ckv.stride(0) if ckv is not None else 0,
-                 ckv.shape[1] if ckv is not None else 1, ptr(app["k_raw"].reshape(B, -1).contiguous()),
-                 ptr(app["k_norm"].to(torch.bfloat16).contiguous()), ptr(kbf),
+                 ckv.shape[1] if ckv is not None else 1, ptr(k_raw), ptr(k_norm), ptr(kbf),
                  kbf.stride(0) if kbf is not None else 0, ptr(k8), k8.stride(0), ptr(ks), ks.stride(0), k8.shape[1],
                  ptr(pos), ptr(seq), ptr(nw), B, int(app["ratio"]), ptr(app["cos"]), ptr(app["sin"]),
-                 int(app["rd"]), float(app["eps"]), ptr(q_idx.contiguous()), ptr(w_idx.to(torch.bfloat16).contiguous()), HI, ptr(cl),
+                 int(app["rd"]), float(app["eps"]), ptr(q_idx), ptr(w_idx), HI, ptr(cl),
                  self.n_pos, ptr(self.score), self.score.stride(0), ptr(self.ws), cp, cs, stream(dev))
             return self.select(cl)
         cp, cs = _cand_args(cand, self.rows, self.n_sel)
-        call("dsv41_decode_select", ptr(x), ptr(app["kv_norm"].to(torch.bfloat16).contiguous()), ptr(ring),
+        call("dsv41_decode_select", ptr(x), ptr(kv_norm), ptr(ring),
              ring.stride(0), ring.shape[1], Dw, ptr(lat), ptr(ckv), ckv.stride(0) if ckv is not None else 0,
-             ckv.shape[1] if ckv is not None else 1, ptr(app["k_raw"].reshape(B, -1).contiguous()),
-             ptr(app["k_norm"].to(torch.bfloat16).contiguous()), ptr(kbf), kbf.stride(0) if kbf is not None else 0,
+             ckv.shape[1] if ckv is not None else 1, ptr(k_raw),
+             ptr(k_norm), ptr(kbf), kbf.stride(0) if kbf is not None else 0,
              ptr(k8), k8.stride(0), ptr(ks), ks.stride(0), k8.shape[1], ptr(pos), ptr(seq), ptr(nw), B,
              int(app["ratio"]), ptr(app["cos"]), ptr(app["sin"]), int(app["rd"]), float(app["eps"]),
-             ptr(q_idx.contiguous()),
-             ptr(w_idx.to(torch.bfloat16).contiguous()), HI, ptr(cl), self.n_sel, self.k, 0, ptr(self.fws),
+             ptr(q_idx), ptr(w_idx), HI, ptr(cl), self.n_sel, self.k, 0, ptr(self.fws),
              self.fnbytes, ptr(self.score) if self.keep_scores else None, self.score.stride(0), ptr(self.out), self.k,
              cp, cs, stream(dev))
         if _lib.CHECK_ERRORS:
@@ -191,8 +192,8 @@ class DecodeSelector:
 
     def __call__(self, q, index_k, weights, seq, cl, k_scale=None, prepared=None, cand=None) -> torch.Tensor:
         dev = require_gpu(q, index_k, weights)
-        seq = as_i64(seq.reshape(-1), dev)
-        cl = as_i64(cl.reshape(-1), dev)
+        seq = as_i64(seq, dev)
+        cl = as_i64(cl, dev)
         if self.one_launch and index_k.dtype == torch.float8_e4m3fn and k_scale is not None:
             if q.shape[0] != self.rows or index_k.shape[1] != self.n_pos:
                 raise RuntimeError(f"DecodeSelector built for {self.rows} x {self.n_pos}, got {q.shape[0]} x "

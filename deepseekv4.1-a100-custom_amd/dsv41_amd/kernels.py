@@ -3,7 +3,7 @@ from __future__ import annotations
 
 import torch
 
-from ._lib import call, ptr, require_gpu, stream
+from ._lib import as_f32, call, ptr, require_gpu, stream
 
 
 def sparse_attn(q: torch.Tensor, kv: torch.Tensor, attn_sink: torch.Tensor, topk_idxs: torch.Tensor,
@@ -27,7 +27,7 @@ def sparse_attn(q: torch.Tensor, kv: torch.Tensor, attn_sink: torch.Tensor, topk
     if kv2 is None or idx.stride(-1) != 1 or idx.stride(-2) < idx.shape[-1] or idx.stride(0) != idx.stride(-2) * s:
         idx = idx.contiguous()
     t = idx.shape[-1]
-    sink = attn_sink.float().contiguous()
+    sink = as_f32(attn_sink)
     out = torch.empty(b, s, h, dv, device=dev, dtype=q.dtype)
     if b * s == 0:
         return out

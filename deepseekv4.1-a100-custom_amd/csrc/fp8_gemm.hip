@@ -28,7 +28,17 @@ constexpr int kGemmLdsBf16 = 32 * 1024;       // staged x elements at most (64 K
 constexpr int kPreMaxK = 2 * kGemmThreads * 32;  // prologue rows: two 32-element groups per thread
 constexpr int kPermK[16] = {0, 1, 8, 9, 2, 3, 10, 11, 4, 5, 12, 13, 6, 7, 14, 15};  // dsv41/w8.py:23
 
-typedef __bf16 bf16x2g_t __attribute__((ext_vector_type(2)));
+typedef float f32x2v_t __attribute__((ext_vector_type(2)));
+
+// fq_value mode 0 of two values by the conversion to e4m3 and back (bit-equal: x / s + 0 gives a negative zero the
+// positive sign round_e4m3 gives it); s a power of two.
+DSV41_DEV f32x2v_t fq8_pair(float a, float b, float s) {
+  const float rs = __int_as_float(0x7f000000 - __float_as_int(s));
+  const float x = fminf(fmaxf(__builtin_fmaf(a, rs, 0.0f), -448.0f), 448.0f);
+  const float y = fminf(fmaxf(__builtin_fmaf(b, rs, 0.0f), -448.0f), 448.0f);
+  const f32x2v_t q = __builtin_amdgcn_cvt_pk_f32_fp8(__builtin_amdgcn_cvt_pk_fp8_f32(x, y, 0, false), false);
+  return f32x2v_t{q.x * s, q.y * s};
+}
 
 struct GemmArgs {
   const uint16_t* x;  // bf16 rows, row stride ldx
@@ -90,94 +100,79 @@ __global__ void __launch_bounds__(kGemmThreads) fp8_gemm_kernel(const GemmArgs a
   load_batch(0, wv, sv);
 
   // ---- stage x[rows, k0..k1) into LDS in the weights' byte order (16-byte units: 8 elements = one half group)
+  // (chunk c of 8 elements of a row's 64 sits at c ^ (row & 7): the rows' strides are multiples of 128 bytes)
+  auto xs_at = [&](int m, int p) { return xs + m * kl + (p & ~63) + ((((p >> 3) & 7) ^ (m & 7)) << 3); };
   if constexpr (PRE) {  // one row, the prologue applied while staging (the arithmetic of dsv41_norm_quant)
+    // 8 elements per thread and step, a scale block in 4 lanes (with a whole block per thread, as norm_quant has it,
+    // 1280 elements kept 40 of 256 threads busy: wq_b 14.5 -> 12.4 us, wo_b 15.7 -> 13.9 us)
     __shared__ float red[kGemmThreads / 64];
-    // 32 x values (raw bf16 pairs) of one group, normalised with its norm weights (mode 1) and fake-quantised, into
-    // LDS at dst in the weights' byte order
-    auto finish = [&](const uint4 (&rx)[4], const uint4 (&rw)[4], float inv, uint16_t* dst) {
-      float v[32];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const uint32_t xx[4] = {rx[q].x, rx[q].y, rx[q].z, rx[q].w};
-        const uint32_t ww[4] = {rw[q].x, rw[q].y, rw[q].z, rw[q].w};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          v[8 * q + 2 * e] = __uint_as_float(xx[e] << 16);
-          v[8 * q + 2 * e + 1] = __uint_as_float(xx[e] & 0xffff0000u);
-          if (a.pre == 1) {
-            v[8 * q + 2 * e] = round_bf16(v[8 * q + 2 * e] * inv * __uint_as_float(ww[e] << 16));
-            v[8 * q + 2 * e + 1] = round_bf16(v[8 * q + 2 * e + 1] * inv * __uint_as_float(ww[e] & 0xffff0000u));
-          }
-        }
-      }
-      float amax = 0.0f;
-#pragma unroll
-      for (int e = 0; e < 32; ++e) amax = fmaxf(amax, fabsf(v[e]));
-      const float sc = fq_scale(amax, 0);
-      const float rs = __fdiv_rn(1.0f, sc);  // sc is a power of two: x * rs == x / sc exactly
-      uint16_t b[32];
-#pragma unroll
-      for (int e = 0; e < 32; ++e) b[e] = f2bf(round_e4m3(fminf(fmaxf(v[e] * rs, -448.0f), 448.0f)) * sc);
-      uint32_t o[16];  // position p of each 16-k group holds k = kPermK[p]
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int j2 = 0; j2 < 8; ++j2)
-          o[8 * h + j2] = (uint32_t)b[16 * h + kPermK[2 * j2]] | ((uint32_t)b[16 * h + kPermK[2 * j2 + 1]] << 16);
-#pragma unroll
-      for (int q = 0; q < 4; ++q) *(uint4*)(dst + 8 * q) = make_uint4(o[4 * q], o[4 * q + 1], o[4 * q + 2], o[4 * q + 3]);
+    const int units = kl / 8;
+    uint4 rx = make_uint4(0, 0, 0, 0), rw = rx;
+    auto load_unit = [&](int u) {
+      rx = *(const uint4*)(a.x + k0 + 8 * u);
+      if (a.pre == 1) rw = *(const uint4*)(a.norm_w + k0 + 8 * u);
     };
-    auto load_grp = [&](int grp, uint4 (&rx)[4], uint4 (&rw)[4]) {  // x and (mode 1) norm weights of a group
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        rx[q] = ((const uint4*)(a.x + 32 * grp))[q];
-        rw[q] = a.pre == 1 ? ((const uint4*)(a.norm_w + 32 * grp))[q] : make_uint4(0, 0, 0, 0);
-      }
-    };
-    const int ng = a.K / 32;
-    const bool whole = k0 == 0 && kl == a.K;  // the slice is the row: the groups loaded for the norm are staged
-    uint4 rx[2][4], rw[2][4];
+    if (tid < units) load_unit(tid);
     float inv = 1.0f;
-    if (a.pre == 1 || whole) {
-#pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        const int grp = tid + kGemmThreads * q;
-        if (grp < ng) load_grp(grp, rx[q], rw[q]);
-        else
-#pragma unroll
-          for (int e = 0; e < 4; ++e) rx[q][e] = rw[q][e] = make_uint4(0, 0, 0, 0);
-      }
-    }
     if (a.pre == 1) {  // whole-row sum of squares, in the order of the norm_quant kernel
       float ss = 0.0f;
 #pragma unroll
-      for (int q = 0; q < 2; ++q)
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const uint32_t xx[4] = {rx[q][u].x, rx[q][u].y, rx[q][u].z, rx[q][u].w};
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const float lo = __uint_as_float(xx[e] << 16), hi = __uint_as_float(xx[e] & 0xffff0000u);
-            ss += lo * lo;
-            ss += hi * hi;
-          }
-        }
-      ss = block_sum<kGemmThreads>(ss, red);
-      inv = __fdiv_rn(1.0f, __fsqrt_rn(__fdiv_rn(ss, (float)a.K) + a.eps));
-    }
-    if (whole) {
-#pragma unroll
       for (int q = 0; q < 2; ++q) {
         const int grp = tid + kGemmThreads * q;
-        if (grp < ng) finish(rx[q], rw[q], inv, xs + 32 * grp);
+        if (grp < a.K / 32) {
+          uint4 r[4];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) r[u] = ((const uint4*)(a.x + 32 * grp))[u];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            const uint32_t xx[4] = {r[u].x, r[u].y, r[u].z, r[u].w};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const float lo = __uint_as_float(xx[e] << 16), hi = __uint_as_float(xx[e] & 0xffff0000u);
+              ss += lo * lo;
+              ss += hi * hi;
+            }
+          }
+        }
       }
-    } else {
+      ss = block_sum<kGemmThreads, true>(ss, red);
+      inv = __fdiv_rn(1.0f, __fsqrt_rn(__fdiv_rn(ss, (float)a.K) + a.eps));
+    }
 #pragma unroll 1
-      for (int u = tid; u < kl / 32; u += kGemmThreads) {
-        uint4 gx[4], gw[4];
-        load_grp(k0 / 32 + u, gx, gw);
-        finish(gx, gw, inv, xs + 32 * u);
+    for (int u = tid; u < units; u += kGemmThreads) {  // (units: a multiple of 8, so whole scale blocks)
+      if (u != tid) load_unit(u);
+      const uint32_t xx[4] = {rx.x, rx.y, rx.z, rx.w}, ww[4] = {rw.x, rw.y, rw.z, rw.w};
+      float v[8], amax = 0.0f;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        v[2 * e] = __uint_as_float(xx[e] << 16);
+        v[2 * e + 1] = __uint_as_float(xx[e] & 0xffff0000u);
+        if (a.pre == 1) {
+          v[2 * e] = round_bf16(v[2 * e] * inv * __uint_as_float(ww[e] << 16));
+          v[2 * e + 1] = round_bf16(v[2 * e + 1] * inv * __uint_as_float(ww[e] & 0xffff0000u));
+        }
+        amax = fmaxf(amax, fmaxf(fabsf(v[2 * e]), fabsf(v[2 * e + 1])));
       }
+      amax = group_max(amax, 4);
+      const float sc = fq_scale(amax, 0);
+      // byte order of a 16-k group: its dwords hold pairs 0 4 1 5 2 6 3 7, so half h's pairs go to dwords 2 e + h
+      uint32_t* dst = (uint32_t*)(xs + 16 * (u >> 1)) + (u & 1);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const f32x2v_t q = fq8_pair(v[2 * e], v[2 * e + 1], sc);
+        dst[2 * e] = (uint32_t)f2bf(q.x) | ((uint32_t)f2bf(q.y) << 16);
+      }
+    }
+  } else if (((uintptr_t)a.x & 15) == 0 && a.ldx % 8 == 0) {
+    // whole 16-k groups in 16-byte units: dword i of the byte order is pair i / 2 of half i & 1
+    const int groups = a.M * (kl / 16);
+#pragma unroll 2
+    for (int u = tid; u < groups; u += kGemmThreads) {
+      const int m = u / (kl / 16), p16 = (u - m * (kl / 16)) * 16;
+      const uint4* src = (const uint4*)(a.x + (long)((a.m0 + m) * xr_mul + xr_off) * a.ldx + k0 + p16);
+      const uint4 lo = src[0], hi = src[1];
+      *(uint4*)xs_at(m, p16) = make_uint4(lo.x, hi.x, lo.y, hi.y);
+      *(uint4*)xs_at(m, p16 + 8) = make_uint4(lo.z, hi.z, lo.w, hi.w);
     }
   } else {
     const int units = a.M * (kl / 8);
@@ -190,7 +185,7 @@ __global__ void __launch_bounds__(kGemmThreads) fp8_gemm_kernel(const GemmArgs a
       const int h = (p8 & 8) ? 8 : 0;  // positions h..h+7 of the group hold k = kPermK[h..h+7]: pairs (2j, 2j+1)
 #pragma unroll
       for (int j = 0; j < 4; ++j) v[j] = *(const uint32_t*)(xrow + kPermK[h + 2 * j]);
-      *(uint4*)(xs + m * kl + p8) = make_uint4(v[0], v[1], v[2], v[3]);
+      *(uint4*)xs_at(m, p8) = make_uint4(v[0], v[1], v[2], v[3]);
     }
   }
   __syncthreads();
@@ -217,10 +212,10 @@ __global__ void __launch_bounds__(kGemmThreads) fp8_gemm_kernel(const GemmArgs a
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) {  // (rows past M: zero operands, nothing staged)
         const bool rv = 16 * mt + l16 < a.M;
-        const uint16_t* xa = xs + (rv ? 16 * mt + l16 : 0) * kl + p;
+        const int m = rv ? 16 * mt + l16 : 0;
         const uint4 z = make_uint4(0, 0, 0, 0);
-        acc[mt] = mfma_bf16_16x16x32(rv ? *(const uint4*)xa : z, b0, acc[mt]);
-        acc[mt] = mfma_bf16_16x16x32(rv ? *(const uint4*)(xa + 8) : z, b1, acc[mt]);
+        acc[mt] = mfma_bf16_16x16x32(rv ? *(const uint4*)xs_at(m, p) : z, b0, acc[mt]);
+        acc[mt] = mfma_bf16_16x16x32(rv ? *(const uint4*)xs_at(m, p + 8) : z, b1, acc[mt]);
       }
     }
 #pragma unroll
@@ -363,14 +358,24 @@ __global__ void __launch_bounds__(kNarrowThreads) fp8_gemv_narrow_kernel(const G
 // thread t of a column takes the 16-k groups t, t + 256 / CPW, ... (every load of the thread in flight at once,
 // up to kVecG groups per batch): 16 weight bytes decoded to fp32 with the block scale (v_cvt_scalef32_pk_f32_fp8,
 // exact) against the group's 16 x elements, then the column's threads reduce (wave shuffles, then LDS; fixed
-// order).  Spreads a small weight over every CU: each workgroup streams CPW x K bytes.
+// order).  Spreads a small weight over every CU: each workgroup streams CPW x K bytes.  x rows are loaded in 16-byte
+// units at their own (4-byte) alignment.
+// PRE (one row): the activation prologue of fp8_gemm_kernel in registers -- a scale block is two threads' groups --
+// while the weights are in flight, the same x as dsv41_norm_quant gives.  Against the 64-column kernel, whose K
+// slices meet in memory: [1280 x 5120] 11.5 -> 7.9 us, [512 x 5120] 9.2 -> 4.6 us.
 constexpr int kVecThreads = 256;
 constexpr int kVecG = 4;
 constexpr int kVecMaxM = 4;
-typedef float f32x2v_t __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4a_t __attribute__((ext_vector_type(4), aligned(4)));
 
-template <int CPW>
+DSV41_DEV uint4 load16_a4(const uint16_t* p) {  // 16 bytes, 4-byte aligned
+  const u32x4a_t v = *(const u32x4a_t*)p;
+  return make_uint4(v.x, v.y, v.z, v.w);
+}
+
+template <int CPW, bool PRE = false>
 __global__ void __launch_bounds__(kVecThreads) fp8_gemv_vec_kernel(const GemmArgs a) {
+  constexpr int MM = PRE ? 1 : kVecMaxM;
   constexpr int TPC = kVecThreads / CPW;    // threads per column
   constexpr int WPC = TPC >= 64 ? TPC / 64 : 1;  // waves per column (a wave holds 64 / TPC columns below 64)
   constexpr int SH = TPC >= 64 ? 64 : TPC;  // lanes of one column inside a wave
@@ -383,17 +388,16 @@ __global__ void __launch_bounds__(kVecThreads) fp8_gemv_vec_kernel(const GemmArg
   const int xr_mul = a.group_cols > 0 ? a.N / a.group_cols : 1;
   const uint8_t* wrow = a.w8 + (long)nc * a.K;
   const uint8_t* srow = a.s8 + (long)(nc >> 5) * a.Kc;
-  const uint16_t* xrow[kVecMaxM];
+  const uint16_t* xrow[MM];
 #pragma unroll
-  for (int m = 0; m < kVecMaxM; ++m)
+  for (int m = 0; m < MM; ++m)
     xrow[m] = a.x + (long)((a.m0 + (m < a.M ? m : 0)) * xr_mul + xr_off) * a.ldx;
   const int ng = a.K / 16;
   const int mine = ng > t ? (ng - t + TPC - 1) / TPC : 0;
   float acc[kVecMaxM] = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll 1
-  for (int j0 = 0; j0 < mine; j0 += kVecG) {
-    uint4 wv[kVecG], xv[kVecG][kVecMaxM][2];
-    uint32_t sv[kVecG];
+  uint4 wv[kVecG], xv[kVecG][MM][2], nv[PRE ? kVecG : 1][2];
+  uint32_t sv[kVecG];
+  auto load = [&](int j0) {
 #pragma unroll
     for (int u = 0; u < kVecG; ++u) {
       const int j = j0 + u < mine ? j0 + u : mine - 1;
@@ -401,16 +405,86 @@ __global__ void __launch_bounds__(kVecThreads) fp8_gemv_vec_kernel(const GemmArg
       wv[u] = *(const uint4*)(wrow + 16 * grp);
       sv[u] = srow[grp >> 1];
 #pragma unroll
-      for (int m = 0; m < kVecMaxM; ++m)
+      for (int m = 0; m < MM; ++m)
         if (m < a.M) {
-          xv[u][m][0] = *(const uint4*)(xrow[m] + 16 * grp);
-          xv[u][m][1] = *(const uint4*)(xrow[m] + 16 * grp + 8);
+          xv[u][m][0] = load16_a4(xrow[m] + 16 * grp);
+          xv[u][m][1] = load16_a4(xrow[m] + 16 * grp + 8);
         }
+      if constexpr (PRE) {
+        if (a.pre == 1) {
+          nv[u][0] = *(const uint4*)(a.norm_w + 16 * grp);
+          nv[u][1] = *(const uint4*)(a.norm_w + 16 * grp + 8);
+        }
+      }
     }
+  };
+  float inv = 1.0f;
+  if constexpr (PRE) {
+    if (a.pre == 1) {  // whole-row sum of squares, in the order of the norm_quant kernel
+      __shared__ float nred[kVecThreads / 64];
+      float ss = 0.0f;
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const int grp = tid + kVecThreads * q;
+        if (grp < a.K / 32) {
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            const uint4 r = ((const uint4*)(a.x + 32 * grp))[u];
+            const uint32_t xx[4] = {r.x, r.y, r.z, r.w};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const float lo = __uint_as_float(xx[e] << 16), hi = __uint_as_float(xx[e] & 0xffff0000u);
+              ss += lo * lo;
+              ss += hi * hi;
+            }
+          }
+        }
+      }
+      if (mine > 0) load(0);  // (in flight over the reduction)
+      ss = block_sum<kVecThreads, true>(ss, nred);
+      inv = __fdiv_rn(1.0f, __fsqrt_rn(__fdiv_rn(ss, (float)a.K) + a.eps));
+    } else if (mine > 0) {
+      load(0);
+    }
+  }
+#pragma unroll 1
+  for (int j0 = 0; j0 < mine; j0 += kVecG) {
+    if (!PRE || j0 > 0) load(j0);
 #pragma unroll
     for (int u = 0; u < kVecG; ++u) {
       if (j0 + u >= mine) break;
       const float sc = e8m0_scale(sv[u]);
+      auto xval = [&](int m, int e) {  // x element e of the group, row m
+        const uint32_t* xw = (const uint32_t*)&xv[u][m][e >> 3];
+        const uint32_t p = xw[(e & 7) >> 1];
+        return __uint_as_float(e & 1 ? p & 0xffff0000u : p << 16);
+      };
+      float xf[16];  // (PRE) the prologue's
+      if constexpr (PRE) {
+        if (a.pre == 1) {
+          const uint32_t ww[8] = {nv[u][0].x, nv[u][0].y, nv[u][0].z, nv[u][0].w,
+                                  nv[u][1].x, nv[u][1].y, nv[u][1].z, nv[u][1].w};
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            xf[2 * i] = round_bf16(xval(0, 2 * i) * inv * __uint_as_float(ww[i] << 16));
+            xf[2 * i + 1] = round_bf16(xval(0, 2 * i + 1) * inv * __uint_as_float(ww[i] & 0xffff0000u));
+          }
+        } else {
+#pragma unroll
+          for (int e = 0; e < 16; ++e) xf[e] = xval(0, e);
+        }
+        float amax = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) amax = fmaxf(amax, fabsf(xf[e]));
+        amax = group_max(amax, 2);  // (groups 2i and 2i + 1 of a scale block: threads t and t ^ 1)
+        const float qs = fq_scale(amax, 0);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const f32x2v_t q = fq8_pair(xf[2 * i], xf[2 * i + 1], qs);  // (bf16 values already)
+          xf[2 * i] = q.x;
+          xf[2 * i + 1] = q.y;
+        }
+      }
       // weight word i (bytes 4i .. 4i + 3) holds k = (2i, 2i + 1) and (2i + 8, 2i + 9) of the group
       const uint32_t ww[4] = {wv[u].x, wv[u].y, wv[u].z, wv[u].w};
 #pragma unroll
@@ -418,19 +492,16 @@ __global__ void __launch_bounds__(kVecThreads) fp8_gemv_vec_kernel(const GemmArg
         const f32x2v_t lo = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(ww[i], sc, false);
         const f32x2v_t hi = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(ww[i], sc, true);
 #pragma unroll
-        for (int m = 0; m < kVecMaxM; ++m) {
+        for (int m = 0; m < MM; ++m) {
           if (m >= a.M) break;
-          const uint32_t* xw0 = (const uint32_t*)&xv[u][m][0];
-          const uint32_t* xw1 = (const uint32_t*)&xv[u][m][1];
-          const uint32_t pl = xw0[i], ph = xw1[i];  // x pairs (2i, 2i + 1) and (2i + 8, 2i + 9)
-          acc[m] += lo.x * bf2f((uint16_t)pl) + lo.y * bf2f((uint16_t)(pl >> 16)) + hi.x * bf2f((uint16_t)ph) +
-                    hi.y * bf2f((uint16_t)(ph >> 16));
+          auto xe = [&](int e) { return PRE ? xf[e] : xval(m, e); };
+          acc[m] += lo.x * xe(2 * i) + lo.y * xe(2 * i + 1) + hi.x * xe(2 * i + 8) + hi.y * xe(2 * i + 9);
         }
       }
     }
   }
 #pragma unroll
-  for (int m = 0; m < kVecMaxM; ++m) {
+  for (int m = 0; m < MM; ++m) {
     float v = acc[m];
 #pragma unroll
     for (int o = SH / 2; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
@@ -438,9 +509,9 @@ __global__ void __launch_bounds__(kVecThreads) fp8_gemv_vec_kernel(const GemmArg
   }
   if ((t & (SH - 1)) == 0)
 #pragma unroll
-    for (int m = 0; m < kVecMaxM; ++m) red[cl][t / SH][m] = acc[m];
+    for (int m = 0; m < MM; ++m) red[cl][t / SH][m] = acc[m];
   __syncthreads();
-  if (t < kVecMaxM && t < a.M && n < a.N) {
+  if (t < MM && t < a.M && n < a.N) {
     float v = 0.0f;
 #pragma unroll
     for (int w = 0; w < WPC; ++w) v += red[cl][w][t];
@@ -448,6 +519,13 @@ __global__ void __launch_bounds__(kVecThreads) fp8_gemv_vec_kernel(const GemmArg
     a.out[o] = f2bf(v);
     if (a.outf) a.outf[o] = v;
   }
+}
+
+template <bool PRE>
+void vec_launch(const GemmArgs& a, int cpw, int grid, hipStream_t st) {
+  if (cpw == 2) fp8_gemv_vec_kernel<2, PRE><<<grid, kVecThreads, 0, st>>>(a);
+  else if (cpw == 4) fp8_gemv_vec_kernel<4, PRE><<<grid, kVecThreads, 0, st>>>(a);
+  else fp8_gemv_vec_kernel<8, PRE><<<grid, kVecThreads, 0, st>>>(a);
 }
 
 // Plan: row tiles of up to 64 rows (MT = 1, 2, 4), K slices so that the grid holds >= 512 workgroups when K allows
@@ -465,7 +543,7 @@ GemmPlan gemm_plan(int M, int N, int K, bool narrow_ok) {
   // 4.2 us; 64-column split 7.2), <= 2048 four (N = 1280: 6.3 us; narrow 7.6), <= 4096 eight (7.6; narrow 8.3);
   // 2-4 rows N <= 1024 two (N = 512, 4 rows: 5.6 us; split 7.8), beyond that narrow (N = 1280, 4 rows: 8.8; vector 9.6)
   p.vec_cpw = 0;
-  if (narrow_ok && M == 1) p.vec_cpw = N <= 1024 ? 2 : N <= 2048 ? 4 : N <= 4096 ? 8 : 0;
+  if (M == 1) p.vec_cpw = N <= 1024 ? 2 : N <= 2048 ? 4 : N <= 4096 ? 8 : 0;  // (at any x alignment, as its PRE form)
   else if (narrow_ok && M <= kVecMaxM && N <= 1024) p.vec_cpw = 2;
   if (p.vec_cpw) {
     p.narrow = false;
@@ -682,10 +760,7 @@ int dsv41_fp8_gemm(const void* x, long ldx, const void* w8, const void* s8, int 
   if (p.vec_cpw) {
     a.m0 = 0;
     a.M = M;
-    if (p.vec_cpw == 1) fp8_gemv_vec_kernel<1><<<p.ctiles, kVecThreads, 0, st>>>(a);
-    else if (p.vec_cpw == 2) fp8_gemv_vec_kernel<2><<<p.ctiles, kVecThreads, 0, st>>>(a);
-    else if (p.vec_cpw == 4) fp8_gemv_vec_kernel<4><<<p.ctiles, kVecThreads, 0, st>>>(a);
-    else fp8_gemv_vec_kernel<8><<<p.ctiles, kVecThreads, 0, st>>>(a);
+    vec_launch<false>(a, p.vec_cpw, p.ctiles, st);
     DSV41_CHECK_LAUNCH();
     return 0;
   }
@@ -716,7 +791,7 @@ int dsv41_fp8_gemv_m1_pre(const void* x_raw, const void* norm_w, float eps, int 
       !x_raw || !w8 || !s8 || !out || ((uintptr_t)x_raw & 15) != 0 || ((uintptr_t)w8 & 15) != 0 ||
       (mode == 1 && ((uintptr_t)norm_w & 15) != 0))
     return (int)hipErrorInvalidValue;
-  const GemmPlan p = gemm_plan(1, N, K, false);  // the 64-column kernel stages x: the prologue runs there
+  const GemmPlan p = gemm_plan(1, N, K, false);  // the vector kernel, or the 64-column kernel's x staging
   if (p.splits > 1 && (!ws || ws_bytes < dsv41_fp8_gemm_workspace_bytes(1, N, K))) return (int)hipErrorInvalidValue;
   GemmArgs a{};
   a.x = (const uint16_t*)x_raw;
@@ -737,6 +812,11 @@ int dsv41_fp8_gemv_m1_pre(const void* x_raw, const void* norm_w, float eps, int 
   if (p.splits > 1) {
     a.cnt = (int*)ws;
     a.part = (float*)((char*)ws + ((long)p.ctiles * 4 + 15) / 16 * 16);
+  }
+  if (p.vec_cpw) {
+    vec_launch<true>(a, p.vec_cpw, p.ctiles, (hipStream_t)stream);
+    DSV41_CHECK_LAUNCH();
+    return 0;
   }
   fp8_gemm_kernel<1, true><<<dim3(p.ctiles, p.splits), kGemmThreads, (size_t)p.kslice * 2, (hipStream_t)stream>>>(a);
   DSV41_CHECK_LAUNCH();

@@ -1093,6 +1093,30 @@ def test_fp8_gemv_m1_pre(mode, N, K):
     assert (np.abs(got - want) <= 1e-5 * mag + np.abs(want) * 2.0 ** -8 + 1e-30).all()
 
 
+@pytest.mark.parametrize("mode,N,K", [(1, 1280, 5120), (2, 512, 5120), (1, 2048, 64), (2, 4096, 1280), (2, 1, 4160),
+                                      (1, 4097, 1280), (2, 8192, 16384)])
+def test_fp8_gemv_m1_pre_kernels(mode, N, K):
+    """The GEMV with its prologue at the edges of its two kernels (up to 4096 columns in registers, 2 to 8 columns a
+    workgroup, and the 64-column kernel past them), K of one batch and of several: bit-equal to norm_quant followed
+    by the GEMV, and within the fp8_gemm bound of float64 products of that x."""
+    from dsv41_amd.fused import norm_quant
+    from dsv41_amd.w8 import W8, fp8_gemm_tc, fp8_gemv_m1_pre
+    g = torch.Generator(device=DEV).manual_seed(N + K)
+    b = torch.randint(0, 256, (N, K), generator=g, device=DEV, dtype=torch.uint8)
+    b[(b & 0x7F) == 0x7F] = 0x01
+    w = W8(b, torch.randint(110, 130, ((N + 31) // 32, K // 32), generator=g, device=DEV, dtype=torch.uint8))
+    x = (torch.randn(1, K, generator=g, device=DEV) * 3).to(torch.bfloat16)
+    nw = (1 + 0.1 * torch.randn(K, generator=g, device=DEV)).to(torch.bfloat16)
+    print(f"[fp8_gemv_m1_pre] mode {mode} N {N} K {K}", flush=True)
+    got = fp8_gemv_m1_pre(x, w.w8, w.s8, nw if mode == 1 else None, 1e-6, mode)
+    xq = torch.empty(K + 2, device=DEV, dtype=torch.bfloat16)[2:].view(1, K)  # (4-byte aligned: no narrow kernel)
+    xq.copy_(norm_quant(x, nw if mode == 1 else None, 1e-6))
+    assert torch.equal(got, fp8_gemm_tc(xq, w.w8, w.s8))
+    wd = w.bf16().double()
+    want, mag = xq.double() @ wd.t(), xq.double().abs() @ wd.abs().t()
+    assert bool(((got.double() - want).abs() <= 1e-5 * mag + 2 ** -8 * want.abs() * 1.01 + 1e-30).all())
+
+
 def test_index_key_snapshot_conversion():
     """Cache snapshots (dsv41/engine.py:1072-1230): the reference's bf16 index-key table -> e4m3 + per-row scale ==
     the oracle's key encoding bit for bit, and back == the original table exactly for FP4-grid rows (the reference's

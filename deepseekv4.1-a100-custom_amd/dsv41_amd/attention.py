@@ -11,7 +11,8 @@ query side (dsv41/model.py:734-746), composed from the HIP entry points of this 
          concatenates both, :1442-1443), then the inverse rope (:1573); optional o-projection (:1574-1576).
 
 The GEMMs of the projections are either the FP8 block-scaled weights of the checkpoint (W8, dsv41_fp8_gemm) or bf16 /
-fp32 tensors (plain library GEMMs through torch, as the reference's F.linear).  Everything else runs on the HIP
+fp32 tensors (plain library GEMMs through torch, as the reference's F.linear; the compressor's two fp32 projections of
+a long chunk by dsv41_f32_proj2).  Everything else runs on the HIP
 library; nothing here falls back to a CPU path."""
 from __future__ import annotations
 
@@ -19,6 +20,7 @@ import torch
 import torch.nn.functional as F
 
 from . import cache as C
+from ._lib import call, ptr, stream
 from .compressor import compress_pool, new_rings
 from .fused import fake_quant_fp4, fake_quant_fp8, rmsnorm, rope_, rope_dev_
 from .indexer import index_topk
@@ -54,6 +56,26 @@ def indexer_query(x: torch.Tensor, qr: torch.Tensor, wq_b, weights_proj: torch.T
     q = fake_quant_fp4(q, 32)
     weights = F.linear(x, weights_proj) * (head_dim ** -0.5 * n_heads ** -0.5)
     return q, weights
+
+
+def compressor_proj(x: torch.Tensor, wkv: torch.Tensor, wgate: torch.Tensor):
+    """dsv41/model.py:593-600: the compressor's fp32 projections F.linear(x.float(), wkv), F.linear(x.float(), wgate).
+
+    From 2^20 results a weight on (2048 rows of 512 columns, 5120 k: 119 us against the library's 165; 1500 rows 119
+    to 133, 1000 rows 118 to 97) and in the kernel's form -- bf16 x, fp32 weights of whole 128-column tiles and 64-k stages,
+    contiguous and 16-byte aligned -- by the HIP kernel, otherwise by the library."""
+    N, K = wkv.shape[0], x.shape[-1]
+    M = x.numel() // max(K, 1)
+    if (x.is_cuda and M * N >= 1 << 20 and N % 128 == 0 and K % 64 == 0 and K < 1 << 21 and x.dtype == torch.bfloat16
+            and x.is_contiguous() and x.data_ptr() % 16 == 0
+            and all(t.dtype == torch.float32 and t.shape == (N, K) and t.device == x.device and t.is_contiguous()
+                    and t.data_ptr() % 16 == 0 for t in (wkv, wgate))):
+        kv = torch.empty(*x.shape[:-1], N, dtype=torch.float32, device=x.device)
+        gate = torch.empty_like(kv)
+        call("dsv41_f32_proj2", ptr(x), K, ptr(wkv), ptr(wgate), M, N, K, ptr(kv), ptr(gate), stream(x.device))
+        return kv, gate
+    xf = x.float()
+    return F.linear(xf, wkv), F.linear(xf, wgate)
 
 
 class SparseAttention:
@@ -108,9 +130,9 @@ class SparseAttention:
             clen = end // ratio
             if clen > self.ckv.shape[1]:
                 raise RuntimeError(f"SparseAttention: {clen} compressed rows exceed the cache capacity {self.ckv.shape[1]}")
-            xf = x.float()
-            latent = compress_pool(F.linear(xf, w["c_wkv"]), F.linear(xf, w["c_wgate"]), start_pos, ratio,
-                                   self.ring_kv[:b], self.ring_score[:b], w["c_norm_w"], eps)
+            ckv, cscore = compressor_proj(x, w["c_wkv"], w["c_wgate"])
+            latent = compress_pool(ckv, cscore, start_pos, ratio, self.ring_kv[:b], self.ring_score[:b],
+                                   w["c_norm_w"], eps)
             new = latent is not None and latent.shape[1] > 0
             ww = widx.shape[-1]
             kk = min(self.topk, clen)

@@ -105,6 +105,13 @@ int dsv41_compress_pool_prefill(const float* kv, const float* score, long x_rstr
                                 int ring, long start_pos, int n_rows, int D, int ratio, const void* norm_w, float eps,
                                 void* latent, long lat_rstride, int n_groups, void* stream);
 
+/* The compressor's wkv / wgate projections of a prefill chunk (dsv41/model.py:593-600, fp32 F.linear of the bf16
+ * hidden states): out0 = x w0^T, out1 = x w1^T, fp32 [M, N], from bf16 x [M, K] (row stride ldx) and fp32 weights
+ * [N, K], in one launch.  Exact products, fp32 accumulation.  K % 64 == 0, N % 128 == 0, ldx % 8 == 0; pointers
+ * 16-byte aligned. */
+int dsv41_f32_proj2(const void* x, long ldx, const float* w0, const float* w1, int M, int N, int K, float* out0,
+                    float* out1, void* stream);
+
 /* ------------------------------------------------------------------------------------------------ indexer */
 
 /* fused3.index_score (dsv41/fused3.py:20-62) and the score half of Indexer.__call__ (dsv41/model.py:766-893):

@@ -108,3 +108,42 @@ def test_sparse_attention_layer(e4m3):
     if e4m3:
         dec = layer.k8.view(torch.float8_e4m3fn).float().cpu().numpy() * layer.ks.cpu().numpy()[..., None]
         np.testing.assert_array_equal(dec, host(layer.index_k))
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 128, 64), (127, 128, 128), (129, 256, 192), (300, 512, 5120),
+                                   (2049, 512, 1280), (8200, 128, 64)])
+def test_compressor_projections_split_weights(M, N, K):
+    """dsv41_f32_proj2 (fp32 weights in three bf16 pieces) at the edges of its tiles and of its three-stage pipeline,
+    against float64.  Products are exact, so the bound is that of fp32 sums of 3 K terms: sqrt(3 K) 2^-24 of the
+    magnitudes, under 1e-5.  At the sizes that compressor_proj sends here its error is no larger than the library's.
+    Infinities and NaN come out as the fp32 products have them."""
+    import torch.nn.functional as F
+    from dsv41_amd._lib import call, ptr, stream
+    from dsv41_amd.attention import compressor_proj
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    w0, w1 = (torch.randn(N, K, generator=g, device=DEV) * K ** -0.5 for _ in range(2))
+    w1 *= torch.exp2(torch.randint(-20, 20, (N, 1), generator=g, device=DEV).float())
+    x = torch.randn(M, K, generator=g, device=DEV).to(torch.bfloat16)
+
+    def run(x):
+        out = torch.full((2, M, N), 7.0, device=DEV)
+        call("dsv41_f32_proj2", ptr(x), K, ptr(w0), ptr(w1), M, N, K, ptr(out[0]), ptr(out[1]), stream(x.device))
+        return out
+    got = run(x)
+    for o, w in zip(got, (w0, w1)):
+        want, mag = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+        assert bool(((o - want).abs() <= 1e-5 * mag).all())
+        if M * N >= 1 << 20:
+            assert float((o - want).norm()) <= float((F.linear(x.float(), w) - want).norm())
+    if M * N >= 1 << 20:
+        assert all(torch.equal(a, b) for a, b in zip(compressor_proj(x.view(1, M, K), w0, w1), got[:, None]))
+    w0[5] = w0[5].to(torch.bfloat16).float()  # (pieces of 0)
+    w0[7, 3] = float("inf")
+    w1[9, K - 1] = float("nan")
+    x[M // 2, 1] = float("-inf")
+    x[M - 1, 2] = float("nan")
+    for o, w in zip(run(x), (w0, w1)):
+        want = (x.double() @ w.double().t()).float()
+        bad = ~torch.isfinite(want)
+        assert torch.equal(torch.isnan(o), torch.isnan(want)) and torch.equal(bad, ~torch.isfinite(o))
+        assert torch.equal(o[bad & ~torch.isnan(o)], want[bad & ~torch.isnan(o)])

@@ -10,8 +10,9 @@
 // slower).  Bound: the MFMAs, 48 a wave and stage, and what they wait for of the split: without two of the three
 // pieces the kernel takes half of its time.  One workgroup a CU, so the time is the same from 1 to 256 workgroups.
 // Two weights of 512 columns, 5120 k, against the two library fp32 products and the fp32 copy of x that they need:
-// 3000 rows 121 us (263), 2048 rows 119 (165), 1500 rows 119 (133), 1000 rows 118 (97), 6000 rows 238 (479).  Relative
-// error against 64 bits 7.9e-7 at every size; the library's 1.2e-6 to 1.3e-6 from 300 rows on, 6.4e-7 below.
+// 3000 rows 122 us (265), 2048 rows 120 (167), 1500 rows 120 (137), 1000 rows 119 (98), 6000 rows 243 (483).  Relative
+// error against 64 bits 1.8e-7 at every size (one fp32 chain over all of K, as fast: 7.9e-7); the library's 1.2e-6 to
+// 1.3e-6 from 300 rows on, 6.4e-7 below.
 #include "common.h"
 
 namespace {
@@ -87,11 +88,20 @@ __global__ void __launch_bounds__(512) f32_proj_kernel(const F32ProjArgs a) {
     if (kt + 1 < nk) __builtin_amdgcn_s_waitcnt(vmcnt_imm(LPT));
     else __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
   };
-  f32x4_t acc[MT][CT];
+  f32x4_t acc[MT][CT], sum[MT][CT];  // chains of 256 k, and their sum
 #pragma unroll
   for (int i = 0; i < MT; ++i)
 #pragma unroll
-    for (int j = 0; j < CT; ++j) acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int j = 0; j < CT; ++j) acc[i][j] = sum[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  auto fold = [&]() {
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < CT; ++j) {
+        sum[i][j] += acc[i][j];
+        acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+      }
+  };
   const int xr = wm * (kFpM / WM) + l16, wr = wn * (kFpN / WN) + l16;
   issue(0, 0);
   if (nk > 1) issue(1, 1);
@@ -119,6 +129,7 @@ __global__ void __launch_bounds__(512) f32_proj_kernel(const F32ProjArgs a) {
 #pragma unroll
       for (int h = 0; h < 2; ++h) x[i][h] = *(const uint4*)(u + (xr + 16 * i) * 128 + ((2 * g + h) ^ (xr >> 1 & 7)) * 16);
     if (!late && kt + 2 < nk) issue(kt + 2, bi == 0 ? 2 : bi - 1);
+    if ((kt & 3) == 0) fold();
     uint4 p[CT][2][3];
     auto split = [&](int h) {
 #pragma unroll
@@ -154,6 +165,7 @@ __global__ void __launch_bounds__(512) f32_proj_kernel(const F32ProjArgs a) {
     bi = bi + 1 == kFpBuf ? 0 : bi + 1;
   }
   if (!late) lds_barrier();
+  fold();
   // lane (l16, g) holds rows m = 16 i + l16, columns 16 j + 4 g .. + 3
 #pragma unroll
   for (int i = 0; i < MT; ++i) {
@@ -162,7 +174,7 @@ __global__ void __launch_bounds__(512) f32_proj_kernel(const F32ProjArgs a) {
 #pragma unroll
     for (int j = 0; j < CT; ++j) {
       const int n = n0 + wn * (kFpN / WN) + 16 * j + 4 * g;
-      f32x4_t v = acc[i][j];
+      f32x4_t v = sum[i][j];
       // an infinity has no pieces and meets pieces of 0: a sum that came out as NaN is taken again, as it stands
 #pragma unroll
       for (int e = 0; e < 4; ++e)

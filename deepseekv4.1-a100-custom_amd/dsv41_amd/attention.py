@@ -22,7 +22,7 @@ import torch.nn.functional as F
 from . import cache as C
 from ._lib import call, ptr, stream
 from .compressor import compress_pool, new_rings
-from .fused import fake_quant_fp4, fake_quant_fp8, rmsnorm, rope_, rope_dev_
+from .fused import fake_quant_fp4, fake_quant_fp8, norm_quant, rmsnorm, rope_, rope_dev_
 from .indexer import index_topk
 from .kernels import sparse_attn
 from .w8 import W8, fp8_gemm_tc
@@ -48,7 +48,12 @@ def indexer_query(x: torch.Tensor, qr: torch.Tensor, wq_b, weights_proj: torch.T
     """Indexer.__call__ query side (dsv41/model.py:734-746): q = fake_quant_fp4(rope(linear_fp8(qr, wq_b)), 32) as
     [b, s, n_heads, head_dim] bf16 (rope at start_pos + i, or at the int64 device positions pos [b] + i when given),
     weights = F.linear(x, weights_proj) * (head_dim^-1/2 * n_heads^-1/2) as [b, s, n_heads] bf16."""
-    q = linear_fp8(qr, wq_b).unflatten(-1, (n_heads, head_dim)).contiguous()
+    return _indexer_query(x, fake_quant_fp8(qr, 32), wq_b, weights_proj, cos, sin, rd, start_pos, n_heads, head_dim, pos)
+
+
+def _indexer_query(x, qrq, wq_b, weights_proj, cos, sin, rd, start_pos, n_heads, head_dim=128, pos=None):
+    """indexer_query of a qr that is on the fp8 grid already."""
+    q = linear_w(qrq, wq_b).unflatten(-1, (n_heads, head_dim)).contiguous()
     if pos is None:
         rope_(q, rd, cos, sin, start_pos)
     else:
@@ -61,8 +66,8 @@ def indexer_query(x: torch.Tensor, qr: torch.Tensor, wq_b, weights_proj: torch.T
 def compressor_proj(x: torch.Tensor, wkv: torch.Tensor, wgate: torch.Tensor):
     """dsv41/model.py:593-600: the compressor's fp32 projections F.linear(x.float(), wkv), F.linear(x.float(), wgate).
 
-    From 2^20 results a weight on (2048 rows of 512 columns, 5120 k: 119 us against the library's 165; 1500 rows 119
-    to 133, 1000 rows 118 to 97) and in the kernel's form -- bf16 x, fp32 weights of whole 128-column tiles and 64-k stages,
+    From 2^20 results a weight on (2048 rows of 512 columns, 5120 k: 120 us against the library's 167; 1500 rows 120
+    to 137, 1000 rows 119 to 98) and in the kernel's form -- bf16 x, fp32 weights of whole 128-column tiles and 64-k stages,
     contiguous and 16-byte aligned -- by the HIP kernel, otherwise by the library."""
     N, K = wkv.shape[0], x.shape[-1]
     M = x.numel() // max(K, 1)
@@ -117,10 +122,17 @@ class SparseAttention:
         w = self.w
         b, s, _ = x.shape
         rd, eps = self.rd, self.eps
-        qr = rmsnorm(linear_fp8(x, w["wq_a"]), w["q_norm_w"], eps)
-        q = linear_fp8(qr, w["wq_b"]).unflatten(-1, (self.H, self.D)).contiguous()
+        # x on the fp8 grid once for both of its projections, qr normed and put there in one pass for both of its own:
+        # three launches fewer than a pass a projection, 3000 rows of the layer 1472 -> 1458 us
+        xq = fake_quant_fp8(x, 32)
+        qr = linear_w(xq, w["wq_a"])
+        if qr.shape[-1] > 1024:  # (shorter rows are summed in another order by rmsnorm: its bits stay)
+            qrq = norm_quant(qr, w["q_norm_w"], eps)
+        else:
+            qrq = fake_quant_fp8(rmsnorm(qr, w["q_norm_w"], eps), 32)
+        q = linear_w(qrq, w["wq_b"]).unflatten(-1, (self.H, self.D)).contiguous()
         rope_(q, rd, self.cos, self.sin, start_pos)
-        win_kv, widx = C.window_kv(linear_fp8(x, w["wkv"]), w["kv_norm_w"], eps, self.cos, self.sin, rd, self.ring,
+        win_kv, widx = C.window_kv(linear_w(xq, w["wkv"]), w["kv_norm_w"], eps, self.cos, self.sin, rd, self.ring,
                                    start_pos)
         if not self.ratio:
             o = sparse_attn(q, win_kv, self.sink, widx, self.scale)
@@ -142,8 +154,8 @@ class SparseAttention:
                 if new:  # the indexer's key append precedes its selection (dsv41/model.py:696-732)
                     C.write_index_k(self.index_k, F.linear(latent, w["i_wk"]), w["i_k_norm_w"], eps, start_pos,
                                     ratio, self.cos, self.sin, rd, k8=self.k8, k_scale=self.ks)
-                qi, wi = indexer_query(x, qr, w["i_wq_b"], w["i_weights_proj"], self.cos, self.sin, rd, start_pos,
-                                       self.HI)
+                qi, wi = _indexer_query(x, qrq, w["i_wq_b"], w["i_weights_proj"], self.cos, self.sin, rd, start_pos,
+                                        self.HI)
                 keys, ks = self._keys(b)
                 index_topk(qi, wi, keys, start_pos, ratio, self.topk, win_kv.shape[1], k_scale=ks,
                            out=idx[:, :, ww:])

@@ -147,3 +147,15 @@ def test_compressor_projections_split_weights(M, N, K):
         bad = ~torch.isfinite(want)
         assert torch.equal(torch.isnan(o), torch.isnan(want)) and torch.equal(bad, ~torch.isfinite(o))
         assert torch.equal(o[bad & ~torch.isnan(o)], want[bad & ~torch.isnan(o)])
+
+
+@pytest.mark.parametrize("D", [1056, 1280, 1536, 4096, 16384])
+def test_norm_quant_is_rmsnorm_then_fake_quant(D):
+    """attend() norms and quantises long query latents in one pass: the bits of the two passes."""
+    from dsv41_amd.fused import fake_quant_fp8, norm_quant, rmsnorm
+    g = torch.Generator(device=DEV).manual_seed(D)
+    w = torch.randn(D, generator=g, device=DEV).to(torch.bfloat16)
+    for M, scale in ((1, 1.0), (7, 1e-6), (300, 1e4), (3000, 1.0)):
+        x = (torch.randn(M, D, generator=g, device=DEV) * scale).to(torch.bfloat16)
+        x[M // 2, : D // 2] = 0
+        assert torch.equal(norm_quant(x, w, 1e-6), fake_quant_fp8(rmsnorm(x, w, 1e-6), 32))

@@ -41,10 +41,16 @@ DSV41_DEV void split2(uint32_t u0, uint32_t u1, uint32_t& hi, uint32_t& mid, uin
   lo = __builtin_amdgcn_perm(q1, q0, 0x07060302u);
 }
 
-// The product as it stands, for what has no finite pieces.
+// The product as it stands, for what has no finite pieces; done at the first NaN (it stays one).
 __device__ __attribute__((noinline)) float f32_dot(const uint16_t* x, const float* w, int K) {
   float s = 0.0f;
-  for (int k = 0; k < K; ++k) s = fmaf(__uint_as_float((uint32_t)x[k] << 16), w[k], s);
+  for (int k = 0; k < K && s == s; k += 8) {
+    const uint4 xv = *(const uint4*)(x + k), w0 = *(const uint4*)(w + k), w1 = *(const uint4*)(w + k + 4);
+    const uint32_t xs[4] = {xv.x, xv.y, xv.z, xv.w}, ws[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      s = fmaf(__uint_as_float(e & 1 ? xs[e / 2] & 0xffff0000u : xs[e / 2] << 16), __uint_as_float(ws[e]), s);
+  }
   return s;
 }
 

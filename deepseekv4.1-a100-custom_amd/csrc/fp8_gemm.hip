@@ -683,12 +683,17 @@ int tile_launch(const TileArgs& a, const TilePlan& p, hipStream_t st) {
 
 }  // namespace
 
+// The streaming kernel's partials, and its whole workspace: what a launch that runs on it is refused without (the tile
+// kernels' slices may need more, and give way to it where they do not get it).
+static long stream_part_bytes(const GemmPlan& p, int N) { return p.splits == 1 ? 0 : (long)p.splits * 16 * p.MT * N * 4; }
+static long stream_bytes(const GemmPlan& p, int N) { return (long)p.ctiles * 4 + 12 + stream_part_bytes(p, N); }
+
 extern "C" {
 
 long dsv41_fp8_gemm_workspace_bytes(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   const GemmPlan p = gemm_plan(M, N, K, false);  // the largest need: the narrow kernel uses none
-  long part = p.splits == 1 ? 0 : (long)p.splits * 16 * p.MT * N * 4;
+  long part = stream_part_bytes(p, N);
   for (int f = 0; f < 6; ++f) {  // (every class of group_cols the plan tells apart, with and without the fp32 result)
     const long t = tile_part_bytes(M, N, tile_plan(M, N, K, f % 3 * kGemmCols, f >= 3));
     part = t > part ? t : part;
@@ -737,7 +742,7 @@ int dsv41_fp8_gemm(const void* x, long ldx, const void* w8, const void* s8, int 
   }
   // the narrow kernel loads x in 16-byte units
   const GemmPlan p = gemm_plan(M, N, K, ((uintptr_t)x & 15) == 0 && ldx % 8 == 0);
-  if (p.splits > 1 && (!ws || ws_bytes < dsv41_fp8_gemm_workspace_bytes(M, N, K))) return (int)hipErrorInvalidValue;
+  if (p.splits > 1 && (!ws || ws_bytes < stream_bytes(p, N))) return (int)hipErrorInvalidValue;
   GemmArgs a{};
   a.x = (const uint16_t*)x;
   a.ldx = ldx;
@@ -792,7 +797,7 @@ int dsv41_fp8_gemv_m1_pre(const void* x_raw, const void* norm_w, float eps, int 
       (mode == 1 && ((uintptr_t)norm_w & 15) != 0))
     return (int)hipErrorInvalidValue;
   const GemmPlan p = gemm_plan(1, N, K, false);  // the vector kernel, or the 64-column kernel's x staging
-  if (p.splits > 1 && (!ws || ws_bytes < dsv41_fp8_gemm_workspace_bytes(1, N, K))) return (int)hipErrorInvalidValue;
+  if (p.splits > 1 && (!ws || ws_bytes < stream_bytes(p, N))) return (int)hipErrorInvalidValue;
   GemmArgs a{};
   a.x = (const uint16_t*)x_raw;
   a.ldx = K;

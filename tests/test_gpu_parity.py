@@ -1011,6 +1011,28 @@ def test_fp8_gemm(M, N, K, gc):
         assert (np.abs(got_u - want) <= 1e-5 * mag + 1e-30).all()
 
 
+@pytest.mark.parametrize("pad", [0, 2])
+def test_fp8_gemm_with_the_streaming_kernels_workspace(pad):
+    """300 rows x 512 columns, K 5120: a workspace of the streaming kernel's size (2 621 484 bytes; the tile kernels'
+    slices want 12 288 044) is taken, one byte less is refused."""
+    from dsv41_amd._lib import lib, ptr, stream
+    M, N, K, need = 300, 512, 5120, 2621484
+    g = torch.Generator(device=DEV).manual_seed(5)
+    b = torch.randint(0, 120, (N, K), generator=g, device=DEV, dtype=torch.uint8)
+    s8 = torch.randint(120, 130, (N // 32, K // 32), generator=g, device=DEV, dtype=torch.uint8)
+    x = torch.randn(M, K + pad, generator=g, device=DEV).to(torch.bfloat16)
+    from dsv41_amd.w8 import fp8_gemm_tc
+    assert lib().dsv41_fp8_gemm_workspace_bytes(M, N, K) >= need
+    out = torch.empty(M, N, device=DEV, dtype=torch.bfloat16)
+    ws = torch.zeros(need, dtype=torch.uint8, device=DEV)
+
+    def rc(n):
+        return lib().dsv41_fp8_gemm(ptr(x), K + pad, ptr(b), ptr(s8), M, N, K, K // 32, 0, ptr(out), N, None, ptr(ws), n,
+                                    stream(x.device))
+    assert rc(need - 1) != 0 and rc(need) == 0
+    assert torch.equal(out, fp8_gemm_tc(x[:, :K].contiguous(), b, s8))  # (N <= 512: the same bits on both kernels)
+
+
 @pytest.mark.parametrize("M,N,K,gc", [(17, 1280, 5120, 0), (24, 512, 5120, 0), (33, 200, 640, 0), (64, 100, 192, 0),
                                       (65, 4096, 1280, 0), (100, 4096, 1280, 0), (130, 1024, 512, 128),
                                       (129, 192, 320, 64), (257, 515, 1280, 0), (300, 2048, 1024, 256),

@@ -578,12 +578,10 @@ struct TileShape {
   int bm, bn, ku, wgs;  // rows, columns, units per stage, workgroups a CU holds
   float t1, t2, fix;    // us per 64 k with one / two workgroups on a CU, and per workgroup (fill, epilogue)
 };
-// The times are measured ones (2048 to 24 rows over the projections' shapes).  The 256-row shapes slow down as the
-// grid fills the chip (power): t1 with one CU in hand, t2 with all.
+// The times are measured ones (2048 to 24 rows over the projections' shapes).
 constexpr TileShape kTiles[] = {
-    {32, 64, 4, 1, 0.235f, 0.0f, 2.4f},   {32, 128, 4, 1, 0.30f, 0.0f, 2.4f}, {64, 64, 2, 2, 0.30f, 0.48f, 2.0f},
-    {64, 128, 1, 2, 0.43f, 0.66f, 2.0f},  {128, 128, 1, 2, 0.62f, 1.05f, 2.5f}, {192, 256, 1, 1, 1.03f, 1.18f, 6.0f},
-    {256, 256, 1, 1, 1.27f, 1.68f, 8.0f}};
+    {32, 64, 4, 1, 0.235f, 0.0f, 2.4f},  {32, 128, 4, 1, 0.30f, 0.0f, 2.4f},  {64, 64, 2, 2, 0.30f, 0.48f, 2.0f},
+    {64, 128, 1, 2, 0.43f, 0.66f, 2.0f}, {128, 128, 1, 2, 0.62f, 1.05f, 2.5f}};
 constexpr int kTileShapes = sizeof(kTiles) / sizeof(kTiles[0]);
 // Columns up to which the sums stay the streaming kernel's bit for bit: the kv latents (512 columns), whose rows go on
 // to the fp8 grid, where a last bit of a sum becomes a whole step.  Cost at 5120 k, us, against the fastest plan and
@@ -598,10 +596,9 @@ struct TilePlan {
   bool same;
 };
 
-// The shape and K slices of the least estimated time: rounds of workgroups over 256 CUs, times their stages, plus the
-// slices' partials written and read and the launch that sums them.  f32: a caller that takes the fp32 sums gets the
-// shapes that keep their chains short.
-TilePlan tile_plan(int M, int N, int K, int group_cols, bool f32) {
+// The shape and K slices of the least estimated time: rounds of workgroups over 256 CUs (an odd last one runs alone
+// on its CU), times their stages, plus the slices' partials written and read and the launch that sums them.
+TilePlan tile_plan(int M, int N, int K, int group_cols) {
   TilePlan best{-1, 1, 0, false};
   if (M < kTileMinM || K > kTileMaxK) return best;
   const int chain = gemm_plan(M, N, K, false).kslice / 64;
@@ -609,18 +606,16 @@ TilePlan tile_plan(int M, int N, int K, int group_cols, bool f32) {
   float tbest = 0.0f;
   for (int c = 0; c < kTileShapes; ++c) {
     const TileShape& t = kTiles[c];
-    if (K % (64 * t.ku) || (group_cols > 0 && group_cols % t.bn) || ((f32 || same) && t.bm > 128) ||
-        (t.bm > 128 && M <= 128) || (same && (c == 1 || chain % t.ku)))
+    if (K % (64 * t.ku) || (group_cols > 0 && group_cols % t.bn) || (same && (c == 1 || chain % t.ku)))
       continue;
     const long tiles = (long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
     const int stages = K / (64 * t.ku), slices = (K / 64 + chain - 1) / chain;
-    for (int s = 1; s <= (same ? slices : 8) && (t.bm <= 128 || s == 1); s = same ? (s < slices ? slices : s + 1) : 2 * s) {
+    for (int s = 1; s <= (same ? slices : 8); s = same ? (s < slices ? slices : s + 1) : 2 * s) {
       if (s > 1 && !same && (stages < 2 * s || (long)s * M * N * 4 > kTilePartMax || tiles * (s / 2) >= 512)) break;
-      const long wg = tiles * s, percu = (wg + 255) / 256, rounds = (percu + t.wgs - 1) / t.wgs;
+      const long percu = (tiles * s + 255) / 256;
       const float units = (float)((stages + s - 1) / s * t.ku);
-      const float fill = wg < 256 ? wg / 256.0f : 1.0f;
-      const float u = t.wgs == 1 ? (t.t2 > 0.0f ? t.t1 + (t.t2 - t.t1) * fill : t.t1) : percu == 1 ? t.t1 : t.t2;
-      float us = rounds * (t.fix + units * u);
+      float us = t.wgs == 1 ? percu * (t.fix + units * t.t1)
+                            : percu / 2 * (t.fix + units * t.t2) + percu % 2 * (t.fix + units * t.t1);
       if (s > 1) us += 3.0f + (float)s * M * N * 8.0f / 4e6f;
       if (best.shape < 0 || us < tbest) {
         best = TilePlan{c, s, chain < t.ku ? t.ku : chain / t.ku * t.ku, same};
@@ -639,7 +634,7 @@ long tile_part_bytes(int M, int N, const TilePlan& p) {
 }
 
 // One launch shape; refuses what its addressing does not take.
-template <int C, int WM, int WN, int NBUF, bool PP, bool SAME>
+template <int C, int WM, int WN, int NBUF, bool SAME>
 int tile_run(TileArgs a, const TilePlan& p, hipStream_t st) {
   constexpr int BM = kTiles[C].bm, BN = kTiles[C].bn, KU = kTiles[C].ku;
   if (a.K % (64 * KU) || a.K > kTileMaxK || (a.group_cols > 0 && a.group_cols % BN) || p.chain % KU ||
@@ -654,7 +649,7 @@ int tile_run(TileArgs a, const TilePlan& p, hipStream_t st) {
   a.ntiles = (a.N + BN - 1) / BN;
   const long tiles = ((long)a.mtiles * a.ntiles + kXcds - 1) / kXcds * kXcds;
   if (tiles >= (1l << 31)) return (int)hipErrorInvalidValue;
-  fp8_tile_kernel<BM, BN, WM, WN, NBUF, KU, PP, SAME>
+  fp8_tile_kernel<BM, BN, WM, WN, NBUF, KU, SAME>
       <<<dim3((unsigned)tiles, a.splits), 64 * WM * WN, 0, st>>>(a);
   DSV41_CHECK_LAUNCH();
   if (a.splits > 1) {
@@ -666,17 +661,15 @@ int tile_run(TileArgs a, const TilePlan& p, hipStream_t st) {
 
 int tile_launch(const TileArgs& a, const TilePlan& p, hipStream_t st) {
   switch (p.shape + 16 * p.same) {
-    case 0: return tile_run<0, 1, 2, 4, false, false>(a, p, st);
-    case 1: return tile_run<1, 1, 4, 3, false, false>(a, p, st);
-    case 2: return tile_run<2, 2, 2, 3, false, false>(a, p, st);
-    case 3: return tile_run<3, 1, 4, 4, false, false>(a, p, st);
-    case 4: return tile_run<4, 2, 2, 3, false, false>(a, p, st);
-    case 5: return tile_run<5, 2, 4, 3, true, false>(a, p, st);
-    case 6: return tile_run<6, 2, 4, 3, true, false>(a, p, st);
-    case 16: return tile_run<0, 1, 2, 4, false, true>(a, p, st);
-    case 18: return tile_run<2, 2, 2, 3, false, true>(a, p, st);
-    case 19: return tile_run<3, 1, 4, 4, false, true>(a, p, st);
-    case 20: return tile_run<4, 2, 2, 3, false, true>(a, p, st);
+    case 0: return tile_run<0, 1, 2, 4, false>(a, p, st);
+    case 1: return tile_run<1, 1, 4, 3, false>(a, p, st);
+    case 2: return tile_run<2, 2, 2, 3, false>(a, p, st);
+    case 3: return tile_run<3, 1, 4, 4, false>(a, p, st);
+    case 4: return tile_run<4, 2, 2, 3, false>(a, p, st);
+    case 16: return tile_run<0, 1, 2, 4, true>(a, p, st);
+    case 18: return tile_run<2, 2, 2, 3, true>(a, p, st);
+    case 19: return tile_run<3, 1, 4, 4, true>(a, p, st);
+    case 20: return tile_run<4, 2, 2, 3, true>(a, p, st);
   }
   return (int)hipErrorInvalidValue;
 }
@@ -694,8 +687,8 @@ long dsv41_fp8_gemm_workspace_bytes(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   const GemmPlan p = gemm_plan(M, N, K, false);  // the largest need: the narrow kernel uses none
   long part = stream_part_bytes(p, N);
-  for (int f = 0; f < 6; ++f) {  // (every class of group_cols the plan tells apart, with and without the fp32 result)
-    const long t = tile_part_bytes(M, N, tile_plan(M, N, K, f % 3 * kGemmCols, f >= 3));
+  for (int f = 0; f < 2; ++f) {  // (both classes of group_cols that the plan tells apart)
+    const long t = tile_part_bytes(M, N, tile_plan(M, N, K, f * kGemmCols));
     part = t > part ? t : part;
   }
   return part ? (long)p.ctiles * 4 + 12 + part : 0;  // counters, pad, partials
@@ -703,8 +696,7 @@ long dsv41_fp8_gemm_workspace_bytes(int M, int N, int K) {
 
 int dsv41_fp8_gemm_tiled(int M, int N, int K, int group_cols) {
   return M > 0 && N > 0 && K > 0 && K % 64 == 0 && tile_rows_ok(K, group_cols > 0 ? N / group_cols : 1) &&
-         tile_plan(M, N, K, group_cols, false).shape >= 0 &&
-         tile_plan(M, N, K, group_cols, true).shape >= 0;
+         tile_plan(M, N, K, group_cols).shape >= 0;
 }
 
 int dsv41_fp8_gemm(const void* x, long ldx, const void* w8, const void* s8, int M, int N, int K, int Kc,
@@ -717,7 +709,7 @@ int dsv41_fp8_gemm(const void* x, long ldx, const void* w8, const void* s8, int 
   const long part0 = ((long)((N + kGemmCols - 1) / kGemmCols) * 4 + 15) / 16 * 16;  // the partials' place in ws
   const long xr_mul = group_cols > 0 ? N / group_cols : 1;
   if (((uintptr_t)x & 15) == 0 && ldx % 8 == 0 && tile_rows_ok(ldx, xr_mul)) {
-    const TilePlan t = tile_plan(M, N, K, group_cols, out_f32 != nullptr);
+    const TilePlan t = tile_plan(M, N, K, group_cols);
     const long need = tile_part_bytes(M, N, t);
     if (t.shape >= 0 && (need == 0 || (ws && ws_bytes >= part0 + need && ((uintptr_t)ws & 15) == 0))) {
       TileArgs a{};

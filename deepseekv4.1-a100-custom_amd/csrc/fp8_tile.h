@@ -20,7 +20,7 @@ struct TileArgs {
   int vec;     // rows of out (and outf) take 4-column stores
   int splits;  // K slices of kslice units (64 k); more than one: fp32 partials [splits, M, ldp] for tile_sum_kernel
   int kslice;
-  int chain;   // units summed in one MFMA chain (not PP); a multiple of the shape's units per stage
+  int chain;   // units summed in one MFMA chain; a multiple of the shape's units per stage
   float* part;
   long ldp;
 };
@@ -57,23 +57,24 @@ DSV41_DEV uint4 tile_decode_b(uint4 w, float sc, int h) {
 
 // WM x WN waves of (BM / WM) rows x (BN / WN) columns; NBUF LDS buffers of KU units of 64 k (128 bytes of an x row,
 // 64 of a weight row each).  The weights are the MFMA's row operand, so a lane ends with 4 adjacent columns of a row.
-//   PP (8 waves, one workgroup per CU, for grids that fill the chip): the two waves of a SIMD alternate, one reads
-//       its operands while the other runs its MFMAs.  256 x 256 keeps a phase MFMA-bound (64 MFMAs against 20 KB of
-//       LDS reads a wave).  Measured, 2048 rows: [8192 x 4096] 107 us (1.28 PFLOP/s; one barrier per stage, both
-//       waves in step: 125 us), [32768 x 1280] 172 us, 256 x 192 for [5120 x 8192] 148 us; the 64-row stream
-//       3119, 3849 and 4672 us.
+// One barrier per stage; two workgroups per CU (one of the 32-row tiles) cover each other's waits, KU > 1 for the small
+// tiles: the chain of barrier, weight read, decode and MFMA is then paid once per KU units; K slices when the tiles
+// leave CUs idle.  Bound: what stands between the MFMAs of a stage (LDS reads, weight decode, the barrier): 2048 rows in
+// 128 x 128 tiles, [32768 x 1280] 237 us, [8192 x 4096] 158 us (0.87 PFLOP/s), [5120 x 8192] 209 us; the 64-row stream
+// 3849, 3119 and 4672 us.
+// Every sum is made of chains as short as the streaming kernel's K slices, so a lane holds its sums twice and 128 x 128
+// is the largest tile.  Not kept: 192 x 256 and 256 x 256 with one chain over all of K, 194, 130 and 180 us, but 1.7e-4,
+// 2.9e-4 and 4.2e-4 of the bf16 results off the rounded product (1.5e-4, 1.9e-4, 2.0e-4 in short chains); 192 x 256 with
+// the second sums as bf16 and the remainder carried on: 230 us and more at equal error.
 //   SAME: the streaming kernel's sums bit for bit: its k order inside an MFMA (8 register moves a 16-row operand; 5 to
 //       10 % of the time) and its K slices as chains.
-//   otherwise one barrier per stage and two workgroups per CU (KU > 1 for the small tiles: the chain of barrier,
-//       weight read, decode and MFMA is then paid once per KU units), with K slices when the tiles leave CUs idle.
-template <int BM, int BN, int WM, int WN, int NBUF, int KU, bool PP, bool SAME>
+template <int BM, int BN, int WM, int WN, int NBUF, int KU, bool SAME>
 __global__ void __launch_bounds__(64 * WM * WN) fp8_tile_kernel(const TileArgs a) {
   constexpr int NT = 64 * WM * WN;
   constexpr int MT = BM / WM / 16, CT = BN / WN / 16;  // 16-row and 16-column tiles of a wave
   constexpr int XB = BM * 128, WB = BN * 64, UNIT = XB + WB;
   constexpr int XL = XB / 16 / NT, WL = WB / 16 / NT, LPT = XL + WL;  // loads per thread and unit
   static_assert(XL * NT * 16 == XB && WL * NT * 16 == WB && (BN / WN) % 32 == 0, "tile shape");
-  static_assert(!PP || (KU == 1 && WM * WN == 8 && NBUF == 3), "two groups of four waves");
   static_assert((NBUF - 2) * KU * LPT < 64, "vmcnt immediate");
   __shared__ __align__(16) uint8_t buf[NBUF * KU * UNIT];
   __shared__ uint8_t scl[BN / 32][kTileMaxK / 32];
@@ -174,75 +175,41 @@ __global__ void __launch_bounds__(64 * WM * WN) fp8_tile_kernel(const TileArgs a
     if (kt + NBUF - 2 < nk) __builtin_amdgcn_s_waitcnt(vmcnt_imm(n));
     else __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
   };
-  int bi = 0;
-  if constexpr (PP) {
-    // phases between barriers: [early: read kt | late: MFMAs kt - 1] [early: MFMAs kt | late: read kt].  Both groups
-    // refill stage kt's buffer (stage kt + NBUF) in the phase after the one in which the late waves read it, and
-    // wait for stage kt + 1's loads before the barrier that ends that reading phase.
-    const bool late = wave >= 4;
-    landed(0);
-    __syncthreads();
-    if (late) {
-      if (NBUF - 1 < nk) issue(NBUF - 1, NBUF - 1);
-      lds_barrier();
-    }
+  // every a.chain units the sums move to a second set, chains as short as the streaming kernel's K slices (fp32
+  // relative error 1.4e-7 at K 1280 in both; in one chain 2.3e-7)
+  int bi = 0, left = 0;
+  f32x4_t tot[MT][CT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < CT; ++j) tot[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll 1
-    for (int kt = 0; kt < nk; ++kt) {
-      Ops o;
-      read(bi, 0, kt, o);
-      if (!late && kt + NBUF - 1 < nk) issue(kt + NBUF - 1, bi == 0 ? NBUF - 1 : bi - 1);
-      if (late) landed(kt + 1);
-      __builtin_amdgcn_sched_barrier(0);
-      lds_barrier();
-      __builtin_amdgcn_sched_barrier(0);
-      if (late && kt + NBUF < nk) issue(kt + NBUF, bi);
-      __builtin_amdgcn_s_setprio(1);
-      mul(o);
-      __builtin_amdgcn_s_setprio(0);
-      if (!late) landed(kt + 1);
-      __builtin_amdgcn_sched_barrier(0);
-      lds_barrier();
-      __builtin_amdgcn_sched_barrier(0);
-      bi = bi + 1 == NBUF ? 0 : bi + 1;
+  for (int kt = 0; kt < nk; ++kt) {
+    landed(kt);
+    lds_barrier();  // stage kt is there for every wave, and every wave has read stage kt - 1
+    if (kt + NBUF - 1 < nk) issue(kt + NBUF - 1, bi == 0 ? NBUF - 1 : bi - 1);
+    if (left == 0) {
+      left = a.chain;
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < CT; ++j) {
+          tot[i][j] += acc[i][j];
+          acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        }
     }
-    if (!late) lds_barrier();
-  } else {
-    // every a.chain units the sums move to a second set, chains as short as the streaming kernel's K slices (fp32
-    // relative error 1.4e-7 at K 1280 in both; in one chain 2.3e-7)
-    int left = 0;
-    f32x4_t tot[MT][CT];
+    Ops o[KU];
 #pragma unroll
-    for (int i = 0; i < MT; ++i)
+    for (int q = 0; q < KU; ++q) read(bi, q, kt * KU + q, o[q]);
 #pragma unroll
-      for (int j = 0; j < CT; ++j) tot[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll 1
-    for (int kt = 0; kt < nk; ++kt) {
-      landed(kt);
-      lds_barrier();  // stage kt is there for every wave, and every wave has read stage kt - 1
-      if (kt + NBUF - 1 < nk) issue(kt + NBUF - 1, bi == 0 ? NBUF - 1 : bi - 1);
-      if (left == 0) {
-        left = a.chain;
-#pragma unroll
-        for (int i = 0; i < MT; ++i)
-#pragma unroll
-          for (int j = 0; j < CT; ++j) {
-            tot[i][j] += acc[i][j];
-            acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-          }
-      }
-      Ops o[KU];
-#pragma unroll
-      for (int q = 0; q < KU; ++q) read(bi, q, kt * KU + q, o[q]);
-#pragma unroll
-      for (int q = 0; q < KU; ++q) mul(o[q]);
-      left -= KU;
-      bi = bi + 1 == NBUF ? 0 : bi + 1;
-    }
-#pragma unroll
-    for (int i = 0; i < MT; ++i)
-#pragma unroll
-      for (int j = 0; j < CT; ++j) acc[i][j] += tot[i][j];
+    for (int q = 0; q < KU; ++q) mul(o[q]);
+    left -= KU;
+    bi = bi + 1 == NBUF ? 0 : bi + 1;
   }
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < CT; ++j) acc[i][j] += tot[i][j];
   // lane (l16, g) holds rows m = 16 i + l16, columns 16 j + 4 g .. + 3
 #pragma unroll
   for (int i = 0; i < MT; ++i) {

@@ -298,7 +298,7 @@ int dsv41_fp8_gemm_tiled(int M, int N, int K, int group_cols);
  * group in the PERM_K byte order; s8: E8M0 [ceil(N / 32), Kc], Kc >= K / 32.  row(m, n) = m, or with group_cols > 0
  * (block-diagonal, dsv41/w8.py oproj_a) m * (N / group_cols) + n / group_cols.  K % 64 == 0; group_cols % 64 == 0;
  * x 4-byte and w8 16-byte aligned.  The weights stream once per 64 rows of M, or (x 16-byte
- * aligned, ldx % 8 == 0, more than 16 rows, K <= 16384) once per up to 256 (the tile kernels).  With x 16-byte aligned and ldx % 8 ==
+ * aligned, ldx % 8 == 0, more than 16 rows, K <= 16384) once per up to 128 (the tile kernels).  With x 16-byte aligned and ldx % 8 ==
  * 0, up to 16 rows over 1024-4096 columns (up to 4 rows over at most 4096 columns, one row there at any alignment of x)
  * run without a K split (faster for the decode GEMVs; the workspace is then unused). */
 int dsv41_fp8_gemm(const void* x, long ldx, const void* w8, const void* s8, int M, int N, int K, int Kc,

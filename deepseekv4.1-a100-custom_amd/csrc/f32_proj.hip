@@ -13,6 +13,8 @@
 // 3000 rows 122 us (265), 2048 rows 120 (167), 1500 rows 120 (137), 1000 rows 119 (98), 6000 rows 243 (483).  Relative
 // error against 64 bits 1.8e-7 at every size (one fp32 chain over all of K, as fast: 7.9e-7); the library's 1.2e-6 to
 // 1.3e-6 from 300 rows on, 6.4e-7 below.
+#include <type_traits>
+
 #include "common.h"
 
 namespace {
@@ -41,17 +43,12 @@ DSV41_DEV void split2(uint32_t u0, uint32_t u1, uint32_t& hi, uint32_t& mid, uin
   lo = __builtin_amdgcn_perm(q1, q0, 0x07060302u);
 }
 
-// The product as it stands, for what has no finite pieces; done at the first NaN (it stays one).
-__device__ __attribute__((noinline)) float f32_dot(const uint16_t* x, const float* w, int K) {
-  float s = 0.0f;
-  for (int k = 0; k < K && s == s; k += 8) {
-    const uint4 xv = *(const uint4*)(x + k), w0 = *(const uint4*)(w + k), w1 = *(const uint4*)(w + k + 4);
-    const uint32_t xs[4] = {xv.x, xv.y, xv.z, xv.w}, ws[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
-#pragma unroll
-    for (int e = 0; e < 8; ++e)
-      s = fmaf(__uint_as_float(e & 1 ? xs[e / 2] & 0xffff0000u : xs[e / 2] << 16), __uint_as_float(ws[e]), s);
-  }
-  return s;
+// A pair of weights as bf16 with every bit that was cut off in the last one: zero, infinite or NaN exactly where the
+// weight is, and of its sign.
+DSV41_DEV uint32_t sticky2(uint32_t u0, uint32_t u1) {
+  u0 |= min(u0 & 0xffffu, 1u) << 16;
+  u1 |= min(u1 & 0xffffu, 1u) << 16;
+  return __builtin_amdgcn_perm(u1, u0, 0x07060302u);
 }
 
 constexpr int kFpM = 128, kFpN = 128, kFpBuf = 3;
@@ -62,6 +59,7 @@ __global__ void __launch_bounds__(512) f32_proj_kernel(const F32ProjArgs a) {
   constexpr int XB = kFpM * 128, WB = kFpN * 256, UNIT = XB + WB;  // bytes of 64 k
   constexpr int XL = XB / 16 / NT, WL = WB / 16 / NT, LPT = XL + WL;
   __shared__ __align__(16) uint8_t buf[kFpBuf * UNIT];
+  __shared__ int again;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int l16 = lane & 15, g = lane >> 4;
   const int wm = wave / WN, wn = wave - wm * WN;
@@ -109,84 +107,113 @@ __global__ void __launch_bounds__(512) f32_proj_kernel(const F32ProjArgs a) {
       }
   };
   const int xr = wm * (kFpM / WM) + l16, wr = wn * (kFpN / WN) + l16;
-  issue(0, 0);
-  if (nk > 1) issue(1, 1);
+  const bool late = wave >= 4;
+  if (tid == 0) again = 0;
+  // One pass over K, into acc and sum; KINDS: with weights of one piece, into acc alone, of which only whether it is
+  // an infinity or NaN is of use.
   // phases between barriers: [early: read kt | late: MFMAs kt - 1] [early: MFMAs kt | late: read kt]; both groups
   // refill stage kt's buffer in the phase after the one in which the late waves read it
-  const bool late = wave >= 4;
-  landed(0);
-  __syncthreads();
-  if (late) {
-    if (nk > 2) issue(2, 2);
-    lds_barrier();
-  }
-  int bi = 0;
+  auto pass = [&](auto kinds) {
+    constexpr bool KINDS = decltype(kinds)::value;
+    issue(0, 0);
+    if (nk > 1) issue(1, 1);
+    landed(0);
+    __syncthreads();
+    if (late) {
+      if (nk > 2) issue(2, 2);
+      lds_barrier();
+    }
+    int bi = 0;
 #pragma unroll 1
-  for (int kt = 0; kt < nk; ++kt) {
-    const uint8_t* u = buf + bi * UNIT;
-    uint4 x[MT][2], w[CT][4];  // k 16 g .. 16 g + 15
+    for (int kt = 0; kt < nk; ++kt) {
+      const uint8_t* u = buf + bi * UNIT;
+      uint4 x[MT][2], w[CT][4];  // k 16 g .. 16 g + 15
+#pragma unroll
+      for (int j = 0; j < CT; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          w[j][q] = *(const uint4*)(u + XB + (wr + 16 * j) * 256 + ((4 * g + q) ^ (wr & 15)) * 16);
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) x[i][h] = *(const uint4*)(u + (xr + 16 * i) * 128 + ((2 * g + h) ^ (xr >> 1 & 7)) * 16);
+      if (!late && kt + 2 < nk) issue(kt + 2, bi == 0 ? 2 : bi - 1);
+      if (!KINDS && (kt & 3) == 0) fold();
+      uint4 p[CT][2][3];
+      auto split = [&](int h) {
+#pragma unroll
+        for (int j = 0; j < CT; ++j) {
+          const uint4 w0 = w[j][2 * h], w1 = w[j][2 * h + 1];
+          if constexpr (KINDS) {
+            p[j][h][0] = make_uint4(sticky2(w0.x, w0.y), sticky2(w0.z, w0.w), sticky2(w1.x, w1.y), sticky2(w1.z, w1.w));
+            continue;
+          }
+          split2(w0.x, w0.y, p[j][h][0].x, p[j][h][1].x, p[j][h][2].x);
+          split2(w0.z, w0.w, p[j][h][0].y, p[j][h][1].y, p[j][h][2].y);
+          split2(w1.x, w1.y, p[j][h][0].z, p[j][h][1].z, p[j][h][2].z);
+          split2(w1.z, w1.w, p[j][h][0].w, p[j][h][1].w, p[j][h][2].w);
+        }
+      };
+      split(0);
+      if (late) landed(kt + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      lds_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      if (late && kt + 3 < nk) issue(kt + 3, bi);
+      __builtin_amdgcn_s_setprio(1);
+      split(1);
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int s = KINDS ? 0 : 2; s >= 0; --s)  // (the small parts first)
+#pragma unroll
+          for (int j = 0; j < CT; ++j)
+#pragma unroll
+            for (int i = 0; i < MT; ++i) acc[i][j] = mfma_bf16_16x16x32(p[j][h][s], x[i][h], acc[i][j]);
+      __builtin_amdgcn_s_setprio(0);
+      if (!late) landed(kt + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      lds_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      bi = bi + 1 == kFpBuf ? 0 : bi + 1;
+    }
+    if (!late) lds_barrier();
+  };
+  pass(std::false_type{});
+  fold();
+  // An infinity has no pieces and meets pieces of 0, so a sum that came out as NaN may be an infinity: a workgroup that
+  // holds one goes over its tile once more for their kinds (3000 rows 125 -> 200 us, wherever and however many they
+  // are; one lane to a sum: 0.35 ms for one infinity, 6.9 ms for a NaN at the end of every row).  A finite result of
+  // that pass says nothing.
+  bool nan = false;
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
 #pragma unroll
     for (int j = 0; j < CT; ++j)
 #pragma unroll
-      for (int q = 0; q < 4; ++q)
-        w[j][q] = *(const uint4*)(u + XB + (wr + 16 * j) * 256 + ((4 * g + q) ^ (wr & 15)) * 16);
+      for (int e = 0; e < 4; ++e) nan |= sum[i][j][e] != sum[i][j][e];
+  if (nan) again = 1;
+  __syncthreads();  // (and every wave is past its last read of the buffers)
+  if (again) {
+    pass(std::true_type{});
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
-      for (int h = 0; h < 2; ++h) x[i][h] = *(const uint4*)(u + (xr + 16 * i) * 128 + ((2 * g + h) ^ (xr >> 1 & 7)) * 16);
-    if (!late && kt + 2 < nk) issue(kt + 2, bi == 0 ? 2 : bi - 1);
-    if ((kt & 3) == 0) fold();
-    uint4 p[CT][2][3];
-    auto split = [&](int h) {
+      for (int j = 0; j < CT; ++j)
 #pragma unroll
-      for (int j = 0; j < CT; ++j) {
-        const uint4 w0 = w[j][2 * h], w1 = w[j][2 * h + 1];
-        split2(w0.x, w0.y, p[j][h][0].x, p[j][h][1].x, p[j][h][2].x);
-        split2(w0.z, w0.w, p[j][h][0].y, p[j][h][1].y, p[j][h][2].y);
-        split2(w1.x, w1.y, p[j][h][0].z, p[j][h][1].z, p[j][h][2].z);
-        split2(w1.z, w1.w, p[j][h][0].w, p[j][h][1].w, p[j][h][2].w);
-      }
-    };
-    split(0);
-    if (late) landed(kt + 1);
-    __builtin_amdgcn_sched_barrier(0);
-    lds_barrier();
-    __builtin_amdgcn_sched_barrier(0);
-    if (late && kt + 3 < nk) issue(kt + 3, bi);
-    __builtin_amdgcn_s_setprio(1);
-    split(1);
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-      for (int s = 2; s >= 0; --s)  // (the small parts first)
-#pragma unroll
-        for (int j = 0; j < CT; ++j)
-#pragma unroll
-          for (int i = 0; i < MT; ++i) acc[i][j] = mfma_bf16_16x16x32(p[j][h][s], x[i][h], acc[i][j]);
-    __builtin_amdgcn_s_setprio(0);
-    if (!late) landed(kt + 1);
-    __builtin_amdgcn_sched_barrier(0);
-    lds_barrier();
-    __builtin_amdgcn_sched_barrier(0);
-    bi = bi + 1 == kFpBuf ? 0 : bi + 1;
+        for (int e = 0; e < 4; ++e) {
+          const float k = acc[i][j][e];
+          if (sum[i][j][e] != sum[i][j][e] && fabsf(k) == __builtin_inff()) sum[i][j][e] = k;
+        }
   }
-  if (!late) lds_barrier();
-  fold();
   // lane (l16, g) holds rows m = 16 i + l16, columns 16 j + 4 g .. + 3
 #pragma unroll
   for (int i = 0; i < MT; ++i) {
     const int m = m0 + wm * (kFpM / WM) + 16 * i + l16;
     if (m >= a.M) continue;
 #pragma unroll
-    for (int j = 0; j < CT; ++j) {
-      const int n = n0 + wn * (kFpN / WN) + 16 * j + 4 * g;
-      f32x4_t v = sum[i][j];
-      // an infinity has no pieces and meets pieces of 0: a sum that came out as NaN is taken again, as it stands
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (v[e] != v[e]) v[e] = f32_dot(a.x + (long)m * a.ldx, a.w[wi] + (long)(n + e) * a.K, a.K);
-      *(f32x4_t*)(a.out[wi] + (long)m * a.N + n) = v;
-    }
+    for (int j = 0; j < CT; ++j)
+      *(f32x4_t*)(a.out[wi] + (long)m * a.N + n0 + wn * (kFpN / WN) + 16 * j + 4 * g) = sum[i][j];
   }
 }
 

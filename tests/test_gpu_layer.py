@@ -149,6 +149,55 @@ def test_compressor_projections_split_weights(M, N, K):
         assert torch.equal(o[bad & ~torch.isnan(o)], want[bad & ~torch.isnan(o)])
 
 
+@pytest.mark.parametrize("M,N,K", [(129, 256, 192), (3000, 512, 5120)])
+def test_compressor_projections_not_finite(M, N, K):
+    """Infinities and NaN wherever they stand come out of dsv41_f32_proj2 as of the products themselves, and take it
+    no more than a second pass: under 3 times the time of finite values (one lane to a sum: 55 times)."""
+    from dsv41_amd._lib import call, ptr, stream
+    g = torch.Generator(device=DEV).manual_seed(M)
+    inf, nan = float("inf"), float("nan")
+    out = torch.empty(2, M, N, device=DEV)
+
+    def run(x, w0, w1):
+        call("dsv41_f32_proj2", ptr(x), K, ptr(w0), ptr(w1), M, N, K, ptr(out[0]), ptr(out[1]), stream(x.device))
+
+    def check(x, w0, w1):
+        run(x, w0, w1)
+        for o, w in zip(out, (w0, w1)):
+            want = (x.double() @ w.double().t()).float()
+            assert torch.equal(torch.isnan(o), torch.isnan(want)) and torch.equal(torch.isinf(o), torch.isinf(want))
+            assert torch.equal(o[torch.isinf(o)], want[torch.isinf(o)])
+
+    def time(x, w0, w1):
+        e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        run(x, w0, w1)
+        e[0].record()
+        for _ in range(4):
+            run(x, w0, w1)
+        e[1].record()
+        torch.cuda.synchronize()
+        return e[0].elapsed_time(e[1])
+
+    x0 = torch.randn(M, K, generator=g, device=DEV).to(torch.bfloat16)
+    w = [torch.randn(N, K, generator=g, device=DEV) * K ** -0.5 for _ in range(2)]
+    w[0][1, K - 1], w[0][2, K - 1], w[0][3, K - 1] = 0.0, 1e-44, -1e-44  # (the two: below bf16's range)
+    w[1][: N // 2] = w[1][: N // 2].to(torch.bfloat16).float()  # (pieces of 0)
+    w[1][5, K - 1] = -inf
+    low = torch.tensor([0x7F800001], dtype=torch.int32, device=DEV).view(torch.float32)  # a NaN in its last bit alone
+    finite = time(x0, w[0], w[0])
+    for v in (inf, -inf, nan):
+        x = x0.clone()
+        x[:, K - 1] = v
+        check(x, *w)
+        assert time(x, *w) < 3 * finite + 0.1
+    x = x0.clone()
+    x[M // 2, 0], x[M // 2, K - 1], x[M - 1, K // 2] = inf, -inf, inf
+    w[0][N - 1, 3] = low
+    check(x, *w)
+    x[:] = nan
+    check(x, *w)
+
+
 @pytest.mark.parametrize("D", [1056, 1280, 1536, 4096, 16384])
 def test_norm_quant_is_rmsnorm_then_fake_quant(D):
     """attend() norms and quantises long query latents in one pass: the bits of the two passes."""

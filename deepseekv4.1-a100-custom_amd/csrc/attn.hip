@@ -1470,7 +1470,8 @@ constexpr int kDecWG = DSV41_DEC_WG;
   // decode-kernel workgroups the split plan aims at
 
 // Split plan.  Decode kernel: <= 192 workgroups over (rows x 16-head groups x splits), >= 2 tiles of 64 keys per
-// split.  64-head kernel: up to 8 splits, one workgroup per CU, when rows are few, >= 3 tiles of 32 keys per split.
+// split.  64-head kernel: one workgroup per CU when rows are few, up to 8 splits (more of long lists), >= 3 tiles of 32
+// keys per split.
 // The 32-head decode kernel's plan (automatic split count only, DV a multiple of 128): splits of 128 keys (64 when that leaves fewer than
 // 96 workgroups), 8 to 64 of them, every workgroup resident at once (one per CU; the head groups of a (row, split) on one
 // XCD).  DSV41_ATTN_DEC32=0 selects the 16-head kernel instead.  Returns false when it does not apply.
@@ -1512,12 +1513,16 @@ void plan(int R, int H, int L, int want, int dv, int* nsplit, int* chunk) {
     const long cus = (long)cus_per_xcd() * kXcds > 0 ? (long)cus_per_xcd() * kXcds : 256;
     const long target = wgs >= cus ? 1 : cus / wgs;
     per = (int)((tiles + target - 1) / target);
-    // up to 8 splits (the combine then loads a row's partials in one round trip: 16 rows x 2176 keys of 576, 8 splits
-    // 27.4 us, 14 30.4 us) of at least 3 tiles (16 rows x 640 keys of 512: 7 splits 26.8 us, 10 29.7 us), and two of
-    // at least 12 (128 rows x 640 keys: one 38.6 us, two 43.7 us)
+    // splits of at least 3 tiles (16 rows x 640 keys of 512: 7 splits 26.8 us, 10 29.7 us); up to 8 of them while they
+    // hold up to 16 tiles each (the combine then loads a row's partials in one round trip: 16 rows x 2176 keys of 576, 8
+    // splits 27.1 us, 14 29.7 us), beyond that up to one round of the rows as the grid pads them (16 rows x 8320 keys
+    // of 512: 8 splits 62.6 us, 16 51.2 us, of 576 52.1 and 45.6; 20 rows: 8 64.5 us, 10 59.9 us, 12, a second round,
+    // 90.8 us); two splits of at least 12 tiles (128 rows x 640 keys of 512: one 43.0 us, two 45.0 us)
     if (target > 1) {
+      const long round = cus / ((R + kXcds - 1) / kXcds * kXcds * ((H + 63) / 64));
+      const int most = tiles > 8 * 16 && round > 8 ? (int)round : 8;
       per = per < 3 ? 3 : per;
-      per = per < (tiles + 7) / 8 ? (tiles + 7) / 8 : per;
+      per = per < (tiles + most - 1) / most ? (tiles + most - 1) / most : per;
       if (target == 2 && per < 12) per = tiles;
     }
   }
@@ -1788,7 +1793,11 @@ int dsv41_sattn2_noalloc(const void* q, const void* kv_win, long win_sstride, in
                        cos_t, sin_t, rd, scale, out, B, h, dv);
   if (rc) return rc;
   a.q_rstride = (long)h * dqk;
-  const long need = dsv41_attn_workspace_bytes(B, h, win + t, dv, want_nsplit);
+  long need = dsv41_attn_workspace_bytes(B, h, win + t, dv, want_nsplit);
+  if (need > DSV41_SCRATCH_BYTES && want_nsplit <= 0 && !use_decode_kernel(B, h)) {  // (8 splits of a long list may fit)
+    want_nsplit = 8;
+    need = dsv41_attn_workspace_bytes(B, h, win + t, dv, want_nsplit);
+  }
   if (need > DSV41_SCRATCH_BYTES) return (int)hipErrorOutOfMemory;  // past the static scratch: pass fewer splits
   void* ws = nullptr;
   if (need > 0) {

@@ -57,7 +57,8 @@ def _rope_tables(rd, n):
 
 # ------------------------------------------------------------------------------------------ many-row attention
 @pytest.mark.parametrize("dqk,R,k,n,nsplit", [(576, 32, 2048, 6000, 0), (576, 48, 300, 250, 0), (512, 24, 512, 9000, 0),
-                                              (512, 16, 512, 700, 1), (512, 40, 130, 4000, 3), (512, 300, 100, 99, 0)])
+                                              (512, 16, 512, 700, 1), (512, 40, 130, 4000, 3), (512, 300, 100, 99, 0),
+                                              (512, 16, 4100, 6000, 0), (576, 16, 4100, 6000, 0)])
 def test_sattn2_many_rows_unit_scale(dqk, R, k, n, nsplit):
     """The 64-head kernel, with (512) and without (576) the inverse rope of the result, at values of unit size against a float64 softmax, three launches bit-equal: gathers still in
     flight when the output is staged would show in single elements.  Rows end in empty entries as short contexts do.

@@ -40,3 +40,16 @@ def test_workspace_query_is_pure():
     assert L.dsv41_attn_workspace_bytes(2048, 64, 2176, 512, 0) == 0  # many rows: one split per row
     n = L.dsv41_attn_workspace_bytes(4, 64, 2176, 512, 0)
     assert n > 0 and n % 4 == 0
+
+
+def test_split_plan_of_many_rows():
+    """Key splits of the 64-head kernel (16 rows x 64 heads and more; 32 keys a tile, fp32 partials of 2 + 512 a split,
+    row and head): 8 at most up to 128 tiles, one round of 256 workgroups over rows padded to 8 beyond, so that a long
+    list is not left to half of the card."""
+    from dsv41_amd._lib import lib
+    for R, H, keys, want in [(16, 64, 640, 7), (16, 64, 2176, 8), (16, 64, 4096, 8), (16, 64, 4224, 15), (16, 64, 8320, 16),
+                             (20, 64, 8320, 10), (24, 64, 8320, 10), (28, 64, 8320, 8), (8, 128, 8320, 16), (9, 128, 8320, 8),
+                             (48, 64, 8320, 5), (128, 64, 640, 1), (128, 64, 768, 2),
+                             (256, 64, 8320, 1)]:
+        n = lib().dsv41_attn_workspace_bytes(R, H, keys, 512, 0)
+        assert (n // (R * H * 514 * 4) if n else 1) == want, (R, H, keys)

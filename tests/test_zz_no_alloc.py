@@ -70,3 +70,21 @@ def test_sattn2_noalloc_matches_workspace_entry():
     torch.cuda.synchronize()
     np.testing.assert_array_equal(out.view(torch.int16).cpu().numpy(), want.view(torch.int16).cpu().numpy())
     assert ctypes.sizeof(ctypes.c_void_p) == 8
+
+
+def test_sattn2_noalloc_long_lists_in_eight_splits():
+    """16 rows x 48 heads x 4224 keys: the library's 15 splits do not fit the static scratch, 8 do and are taken."""
+    from dsv41_amd._lib import lib
+    L = lib()
+    st = torch.cuda.current_stream().cuda_stream
+    g = torch.Generator(device=DEV).manual_seed(72)
+    q, ring, ckv, idx, pos, seq, sink = _inputs(g, 16, 4096, H=48)
+    want = torch.empty(16, 1, 48, 512, dtype=torch.bfloat16, device=DEV)
+    got = torch.full_like(want, 7.0)
+    nbytes = L.dsv41_attn_workspace_bytes(16, 48, 4224, 512, 8)
+    assert nbytes <= 16 << 20 < L.dsv41_attn_workspace_bytes(16, 48, 4224, 512, 0)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=DEV)
+    print("[noalloc] B 16 H 48 t 4096", flush=True)
+    assert L.dsv41_sattn2(*_args(q, ring, ckv, idx, pos, seq, sink, want), 8, ws.data_ptr(), nbytes, st) == 0
+    assert L.dsv41_sattn2_noalloc(*_args(q, ring, ckv, idx, pos, seq, sink, got), 0, st) == 0
+    assert torch.equal(got, want)

@@ -1517,13 +1517,14 @@ void plan(int R, int H, int L, int want, int dv, int* nsplit, int* chunk) {
     // hold up to 16 tiles each (the combine then loads a row's partials in one round trip: 16 rows x 2176 keys of 576, 8
     // splits 27.1 us, 14 29.7 us), beyond that up to one round of the rows as the grid pads them (16 rows x 8320 keys
     // of 512: 8 splits 62.6 us, 16 51.2 us, of 576 52.1 and 45.6; 20 rows: 8 64.5 us, 10 59.9 us, 12, a second round,
-    // 90.8 us); two splits of at least 12 tiles (128 rows x 640 keys of 512: one 43.0 us, two 45.0 us)
+    // 90.8 us); two splits of at least 12 tiles, 10 where the combine has fewer rows (640 keys of 512: 128 rows, one
+    // split 43.0 us, two 45.0 us; 88 rows 42.6 and 40.5 us)
     if (target > 1) {
       const long round = cus / ((R + kXcds - 1) / kXcds * kXcds * ((H + 63) / 64));
       const int most = tiles > 8 * 16 && round > 8 ? (int)round : 8;
       per = per < 3 ? 3 : per;
       per = per < (tiles + most - 1) / most ? (tiles + most - 1) / most : per;
-      if (target == 2 && per < 12) per = tiles;
+      if (target == 2 && per < (wgs > 104 ? 12 : 10)) per = tiles;
     }
   }
   if (per < 1) per = 1;

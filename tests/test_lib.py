@@ -49,7 +49,7 @@ def test_split_plan_of_many_rows():
     from dsv41_amd._lib import lib
     for R, H, keys, want in [(16, 64, 640, 7), (16, 64, 2176, 8), (16, 64, 4096, 8), (16, 64, 4224, 15), (16, 64, 8320, 16),
                              (20, 64, 8320, 10), (24, 64, 8320, 10), (28, 64, 8320, 8), (8, 128, 8320, 16), (9, 128, 8320, 8),
-                             (48, 64, 8320, 5), (128, 64, 640, 1), (128, 64, 768, 2),
+                             (48, 64, 8320, 5), (88, 64, 640, 2), (104, 64, 640, 2), (112, 64, 640, 1), (128, 64, 768, 2),
                              (256, 64, 8320, 1)]:
         n = lib().dsv41_attn_workspace_bytes(R, H, keys, 512, 0)
         assert (n // (R * H * 514 * 4) if n else 1) == want, (R, H, keys)

@@ -366,6 +366,7 @@ __global__ void __launch_bounds__(kNarrowThreads) fp8_gemv_narrow_kernel(const G
 constexpr int kVecThreads = 256;
 constexpr int kVecG = 4;
 constexpr int kVecMaxM = 4;
+constexpr int kVecMaxN = 4096;
 typedef uint32_t u32x4a_t __attribute__((ext_vector_type(4), aligned(4)));
 
 DSV41_DEV uint4 load16_a4(const uint16_t* p) {  // 16 bytes, 4-byte aligned
@@ -536,6 +537,16 @@ struct GemmPlan {
   int vec_cpw;  // > 0: fp8_gemv_vec_kernel with this many columns per workgroup
 };
 
+// One row with its prologue, or at 4-byte alignment: the vector kernel where each of its threads has few groups to put
+// on the grid itself, the 64-column kernel, which does that once a workgroup, elsewhere.  Vector / 64 columns, us, with
+// the norm and without: [1280 x 5120] 11.5 / 10.3 and 7.2 / 9.4, [1280 x 8192] 14.9 / 14.6 and 8.6 / 13.2, [2048 x 8192]
+// 14.8 / 11.4 and 8.9 / 9.9, [4096 x 1280] 8.3 / 7.2 and 5.5 / 6.4, [4096 x 5120] 18.5 / 11.3 and 10.8 / 10.0,
+// [4096 x 16384] 51 / 20 and 29 / 18, [1024 x 16384] 15.6 / 16.0 and 8.8 / 14.0; in one K slice (under 512 k)
+// [1280 x 256] 5.2 / 4.4 and 3.7 / 3.4.
+bool one_row_vec(int N, int K) {
+  return K >= 512 && K <= (N <= 1024 ? 16384 : N <= 1536 ? 8192 : N <= 2048 ? 5120 : 1280);
+}
+
 GemmPlan gemm_plan(int M, int N, int K, bool narrow_ok) {
   GemmPlan p{};
   p.narrow = narrow_ok && M <= 16 && N >= kNarrowMinN && N <= kNarrowMaxN;
@@ -543,7 +554,7 @@ GemmPlan gemm_plan(int M, int N, int K, bool narrow_ok) {
   // 4.2 us; 64-column split 7.2), <= 2048 four (N = 1280: 6.3 us; narrow 7.6), <= 4096 eight (7.6; narrow 8.3);
   // 2-4 rows N <= 1024 two (N = 512, 4 rows: 5.6 us; split 7.8), beyond that narrow (N = 1280, 4 rows: 8.8; vector 9.6)
   p.vec_cpw = 0;
-  if (M == 1) p.vec_cpw = N <= 1024 ? 2 : N <= 2048 ? 4 : N <= 4096 ? 8 : 0;  // (at any x alignment, as its PRE form)
+  if (M == 1 && (narrow_ok || one_row_vec(N, K))) p.vec_cpw = N <= 1024 ? 2 : N <= 2048 ? 4 : N <= kVecMaxN ? 8 : 0;
   else if (narrow_ok && M <= kVecMaxM && N <= 1024) p.vec_cpw = 2;
   if (p.vec_cpw) {
     p.narrow = false;
@@ -733,8 +744,11 @@ int dsv41_fp8_gemm(const void* x, long ldx, const void* w8, const void* s8, int 
     }
   }
   // the narrow kernel loads x in 16-byte units
-  const GemmPlan p = gemm_plan(M, N, K, ((uintptr_t)x & 15) == 0 && ldx % 8 == 0);
-  if (p.splits > 1 && (!ws || ws_bytes < stream_bytes(p, N))) return (int)hipErrorInvalidValue;
+  GemmPlan p = gemm_plan(M, N, K, ((uintptr_t)x & 15) == 0 && ldx % 8 == 0);
+  if (p.splits > 1 && (!ws || ws_bytes < stream_bytes(p, N))) {
+    if (M > 1 || N > kVecMaxN) return (int)hipErrorInvalidValue;
+    p = gemm_plan(1, N, K, true);  // (the vector kernel needs none, and takes any alignment)
+  }
   GemmArgs a{};
   a.x = (const uint16_t*)x;
   a.ldx = ldx;
@@ -788,8 +802,11 @@ int dsv41_fp8_gemv_m1_pre(const void* x_raw, const void* norm_w, float eps, int 
       !x_raw || !w8 || !s8 || !out || ((uintptr_t)x_raw & 15) != 0 || ((uintptr_t)w8 & 15) != 0 ||
       (mode == 1 && ((uintptr_t)norm_w & 15) != 0))
     return (int)hipErrorInvalidValue;
-  const GemmPlan p = gemm_plan(1, N, K, false);  // the vector kernel, or the 64-column kernel's x staging
-  if (p.splits > 1 && (!ws || ws_bytes < stream_bytes(p, N))) return (int)hipErrorInvalidValue;
+  GemmPlan p = gemm_plan(1, N, K, false);  // the vector kernel, or the 64-column kernel's x staging
+  if (p.splits > 1 && (!ws || ws_bytes < stream_bytes(p, N))) {
+    if (N > kVecMaxN) return (int)hipErrorInvalidValue;
+    p = gemm_plan(1, N, K, true);  // (the vector kernel needs none)
+  }
   GemmArgs a{};
   a.x = (const uint16_t*)x_raw;
   a.ldx = K;

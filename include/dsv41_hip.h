@@ -297,18 +297,19 @@ int dsv41_fp8_gemm_tiled(int M, int N, int K, int group_cols);
  * accumulation, bf16 out [M, ldo] (and fp32 out_f32 [M, ldo] when not null).  w8: e4m3 bits [N, K] with every 16-k
  * group in the PERM_K byte order; s8: E8M0 [ceil(N / 32), Kc], Kc >= K / 32.  row(m, n) = m, or with group_cols > 0
  * (block-diagonal, dsv41/w8.py oproj_a) m * (N / group_cols) + n / group_cols.  K % 64 == 0; group_cols % 64 == 0;
- * x 4-byte and w8 16-byte aligned.  The weights stream once per 64 rows of M, or (x 16-byte
- * aligned, ldx % 8 == 0, more than 16 rows, K <= 16384) once per up to 128 (the tile kernels).  With x 16-byte aligned and ldx % 8 ==
- * 0, up to 16 rows over 1024-4096 columns (up to 4 rows over at most 4096 columns, one row there at any alignment of x)
- * run without a K split (faster for the decode GEMVs; the workspace is then unused). */
+ * x 4-byte and w8 16-byte aligned.  The weights stream once per 64 rows of M, or (x 16-byte aligned, ldx % 8 == 0,
+ * more than 16 rows, K <= 16384) once per up to 128 (the tile kernels).  With x 16-byte aligned and ldx % 8 == 0, up to
+ * 16 rows over 1024-4096 columns (up to 4 rows over at most 4096 columns) run without a K split (faster for the decode
+ * GEMVs; the workspace is then unused), as does one row there at any alignment of x for K from 512 up to 16384 / 8192 /
+ * 5120 / 1280 over up to 1024 / 1536 / 2048 / 4096 columns, or without a workspace. */
 int dsv41_fp8_gemm(const void* x, long ldx, const void* w8, const void* s8, int M, int N, int K, int Kc,
                    int group_cols, void* out, long ldo, float* out_f32, void* ws, long ws_bytes, void* stream);
 
 /* fp8_gemv_m1_pre (dsv41/cukern.py:137-158): one launch, the activation prologue fused into the GEMV's x loads:
  * x = fake_quant_fp8(bf16(rmsnorm(x_raw) * norm_w), 32) (mode 1) or fake_quant_fp8(x_raw, 32) (mode 2; norm_w
  * unused), then out[0, n] as dsv41_fp8_gemm for one row.  x_raw bf16 [K] and norm_w 16-byte aligned, K % 64 == 0,
- * K <= 16384; the same results as dsv41_norm_quant followed by dsv41_fp8_gemm (over 4096 columns: on its 64-column
- * kernel, which one row of x at any alignment takes there).  Workspace: dsv41_fp8_gemm_workspace_bytes(1, N, K). */
+ * K <= 16384; the same results as dsv41_norm_quant followed by dsv41_fp8_gemm of one row of x at 4-byte alignment (the
+ * same kernel by the same sizes).  Workspace: dsv41_fp8_gemm_workspace_bytes(1, N, K). */
 int dsv41_fp8_gemv_m1_pre(const void* x_raw, const void* norm_w, float eps, int mode, const void* w8, const void* s8,
                           int N, int K, int Kc, void* out, void* ws, long ws_bytes, void* stream);
 

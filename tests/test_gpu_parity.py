@@ -1149,10 +1149,11 @@ def test_fp8_gemv_m1_pre(mode, N, K):
 
 
 @pytest.mark.parametrize("mode,N,K", [(1, 1280, 5120), (2, 512, 5120), (1, 2048, 64), (2, 4096, 1280), (2, 1, 4160),
-                                      (1, 4097, 1280), (2, 8192, 16384)])
+                                      (1, 4097, 1280), (2, 8192, 16384), (1, 300, 448), (2, 1024, 16384), (1, 1536, 8192),
+                                      (2, 1537, 8192), (1, 4096, 1344), (1, 2048, 5184)])
 def test_fp8_gemv_m1_pre_kernels(mode, N, K):
-    """The GEMV with its prologue at the edges of its two kernels (up to 4096 columns in registers, 2 to 8 columns a
-    workgroup, and the 64-column kernel past them), K of one batch and of several: bit-equal to norm_quant followed
+    """The GEMV with its prologue at the edges of its two kernels (the vector kernel, 2 to 8 columns a workgroup, and the
+    64-column kernel for wider weights, long and short K), K of one batch and of several: bit-equal to norm_quant followed
     by the GEMV, and within the fp8_gemm bound of float64 products of that x."""
     from dsv41_amd.fused import norm_quant
     from dsv41_amd.w8 import W8, fp8_gemm_tc, fp8_gemv_m1_pre
@@ -1170,6 +1171,48 @@ def test_fp8_gemv_m1_pre_kernels(mode, N, K):
     wd = w.bf16().double()
     want, mag = xq.double() @ wd.t(), xq.double().abs() @ wd.abs().t()
     assert bool(((got.double() - want).abs() <= 1e-5 * mag + 2 ** -8 * want.abs() * 1.01 + 1e-30).all())
+
+
+def _graph_us(fn, n=20, reps=10):
+    """The least time of one of n launches in a replayed graph."""
+    fn()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        for _ in range(n):
+            fn()
+    graph.replay()
+    ms = []
+    for _ in range(reps):
+        e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        e[0].record()
+        graph.replay()
+        e[1].record()
+        torch.cuda.synchronize()
+        ms.append(e[0].elapsed_time(e[1]))
+    return min(ms) * 1e3 / n
+
+
+@pytest.mark.parametrize("N,K", [(4096, 5120), (3072, 8192), (4096, 16384), (2048, 16384), (1280, 5120), (300, 64)])
+def test_fp8_gemv_m1_pre_is_no_slower_than_two_launches(N, K):
+    """The prologue in the GEMV's launch against the norm_quant and GEMV launches that it replaces (each column's threads
+    repeating it took twice their time over 4096 columns of 16384 k); and without a workspace the same kernels' results
+    within the rounding of two summation orders."""
+    from dsv41_amd._lib import lib, ptr, stream
+    from dsv41_amd.fused import norm_quant
+    from dsv41_amd.w8 import W8, fp8_gemm_tc, fp8_gemv_m1_pre
+    g = torch.Generator(device=DEV).manual_seed(N + K)
+    w = W8(torch.randint(0, 120, (N, K), generator=g, device=DEV, dtype=torch.uint8),
+           torch.randint(118, 124, ((N + 31) // 32, K // 32), generator=g, device=DEV, dtype=torch.uint8))
+    x, nw = torch.randn(1, K, generator=g, device=DEV).to(torch.bfloat16), torch.ones(K, device=DEV, dtype=torch.bfloat16)
+    one = _graph_us(lambda: fp8_gemv_m1_pre(x, w.w8, w.s8, nw, 1e-6, 1))
+    two = _graph_us(lambda: fp8_gemm_tc(norm_quant(x, nw, 1e-6), w.w8, w.s8))
+    assert one < 1.1 * two, (one, two)
+    out = torch.empty(1, N, device=DEV, dtype=torch.bfloat16)
+    assert lib().dsv41_fp8_gemv_m1_pre(ptr(x), ptr(nw), 1e-6, 1, ptr(w.w8), ptr(w.s8), N, K, K // 32, ptr(out), None, 0,
+                                       stream(x.device)) == 0
+    assert bool(((out.float() - fp8_gemv_m1_pre(x, w.w8, w.s8, nw, 1e-6, 1).float()).abs() <= 2 ** -7 * out.float().abs()
+                 + 1e-5 * (norm_quant(x, nw, 1e-6).float().abs() @ w.bf16().float().abs().t())).all())
 
 
 def test_index_key_snapshot_conversion():

@@ -246,8 +246,11 @@ __global__ void __launch_bounds__(256) index_keys_decode_kernel(const uint8_t* k
 }
 
 // The same conversions for 16-byte aligned tables, bound by memory: 16 lanes per row, 8 values (16 and 8 bytes) per lane,
-// four rows in flight per lane.  262144 rows: encode 45.8 -> 17.4 us (5.9 TB/s), decode 31.5 -> 18.0 us.
+// four rows in flight per lane.  262144 rows: encode 45.8 -> 17.4 us (5.9 TB/s), decode 31.5 -> 18.0 us.  A wave does
+// 16 rows where the kernels above do one, so few rows take longer: encode 4096 rows 3.1 us (2.7 above), 6000 3.1 (3.1),
+// 8192 3.2 (3.4); decode 4096 rows 3.6 us (2.4), 16384 4.0 (3.7), 24576 4.5 (4.5), 32768 4.9 (5.3).
 constexpr int kConvRows = 4;  // rows per 16 lanes, 16 rows apart
+constexpr long kEncode16Rows = 6144, kDecode16Rows = 24576;
 
 __global__ void __launch_bounds__(256) index_keys_encode16_kernel(const uint16_t* kbf, long n_rows, uint8_t* k8,
                                                                   float* ks) {
@@ -592,7 +595,7 @@ int dsv41_decode_appends(const void* kv_raw, const void* kv_norm, void* ring, lo
 int dsv41_index_keys_encode(const void* kbf, long n_rows, void* k8, float* ks, void* stream) {
   if (n_rows <= 0) return 0;
   if (!kbf || !k8 || !ks) return (int)hipErrorInvalidValue;
-  if (((uintptr_t)kbf & 15) == 0 && ((uintptr_t)k8 & 7) == 0) {
+  if (n_rows >= kEncode16Rows && ((uintptr_t)kbf & 15) == 0 && ((uintptr_t)k8 & 7) == 0) {
     index_keys_encode16_kernel<<<(unsigned)((n_rows + 16 * kConvRows - 1) / (16 * kConvRows)), 256, 0,
                                  (hipStream_t)stream>>>((const uint16_t*)kbf, n_rows, (uint8_t*)k8, ks);
     DSV41_CHECK_LAUNCH();
@@ -607,7 +610,7 @@ int dsv41_index_keys_encode(const void* kbf, long n_rows, void* k8, float* ks, v
 int dsv41_index_keys_decode(const void* k8, const float* ks, long n_rows, void* kbf, void* stream) {
   if (n_rows <= 0) return 0;
   if (!kbf || !k8 || !ks) return (int)hipErrorInvalidValue;
-  if (((uintptr_t)kbf & 15) == 0 && ((uintptr_t)k8 & 7) == 0) {
+  if (n_rows >= kDecode16Rows && ((uintptr_t)kbf & 15) == 0 && ((uintptr_t)k8 & 7) == 0) {
     index_keys_decode16_kernel<<<(unsigned)((n_rows + 16 * kConvRows - 1) / (16 * kConvRows)), 256, 0,
                                  (hipStream_t)stream>>>((const uint8_t*)k8, ks, n_rows, (uint16_t*)kbf);
     DSV41_CHECK_LAUNCH();

@@ -129,15 +129,17 @@ def test_row_operations_aligned_and_not(group, mode):
             same(x, y)
 
 
-@pytest.mark.parametrize("n", [1, 63, 64, 1003])
+@pytest.mark.parametrize("n", [1, 63, 64, 1003, 6143, 6145, 24575, 24577])
 def test_index_key_conversion_aligned_and_not(n):
-    """The converters' 16-byte form against the general one (tables at an odd alignment), bit for bit: row remainders,
-    values far below the row's maximum (subnormal codes, zeros of both signs), every byte code."""
+    """The converters' 16-byte form (many rows) against the general one (tables at an odd alignment), bit for bit: row
+    remainders, values far below the row's maximum (subnormal codes, zeros of both signs), infinities and NaN, every
+    byte code."""
     from dsv41_amd._lib import call, ptr, stream
     g = torch.Generator(device=DEV).manual_seed(n)
     k = (torch.randn(n, 128, generator=g, device=DEV) *
          torch.exp2(torch.randint(-24, 4, (n, 128), generator=g, device=DEV).float())).to(torch.bfloat16)
     k[0, :7] = -0.0
+    k[n // 2, 5], k[n // 3, 9], k[n - 1, 127] = float("inf"), float("nan"), float("-inf")
     st = stream(k.device)
     res = []
     for off in (0, 2):
@@ -1191,6 +1193,18 @@ def _graph_us(fn, n=20, reps=10):
         torch.cuda.synchronize()
         ms.append(e[0].elapsed_time(e[1]))
     return min(ms) * 1e3 / n
+
+
+def test_index_key_conversion_of_few_rows():
+    """4096 aligned rows take no longer than unaligned ones, which always go to the general kernels."""
+    from dsv41_amd._lib import call, ptr, stream
+    k = torch.randn(4096 * 128 + 2, device=DEV).to(torch.bfloat16)
+    k8, ks = torch.empty(4096, 128, dtype=torch.uint8, device=DEV), torch.empty(4096, device=DEV)
+    for name in ("dsv41_index_keys_encode", "dsv41_index_keys_decode"):
+        args = lambda x: ((ptr(x), 4096, ptr(k8), ptr(ks)) if "encode" in name else  # noqa: E731
+                          (ptr(k8), ptr(ks), 4096, ptr(x)))
+        us = [_graph_us(lambda x=x: call(name, *args(x), stream(k.device))) for x in (k[:-2], k[2:])]
+        assert us[0] <= 1.08 * us[1], (name, us)
 
 
 @pytest.mark.parametrize("N,K", [(4096, 5120), (3072, 8192), (4096, 16384), (2048, 16384), (1280, 5120), (300, 64)])

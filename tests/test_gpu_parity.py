@@ -115,8 +115,8 @@ def test_row_operations_aligned_and_not(group, mode):
     def same(a, b):
         assert torch.equal(a.view(torch.int16), b.view(torch.int16))
 
-    for D in (group, 96, 576, 1024):
-        x = wide(37, D)
+    for rows, D in ((37, group), (37, 96), (37, 576), (37, 1024), (1403, group), (1401, 96), (501, 512)):
+        x = wide(rows, D)
         x[3, 5], x[4, 7], x[5] = float("inf"), float("nan"), 0.0
         same(dsv41_amd.fake_quant(x, group, mode), dsv41_amd.fake_quant(odd(x), group, mode))
     cos, sin = torch.rand(64, 32, generator=g, device=DEV), torch.rand(64, 32, generator=g, device=DEV)
@@ -1205,6 +1205,18 @@ def test_index_key_conversion_of_few_rows():
                           (ptr(k8), ptr(ks), 4096, ptr(x)))
         us = [_graph_us(lambda x=x: call(name, *args(x), stream(k.device))) for x in (k[:-2], k[2:])]
         assert us[0] <= 1.08 * us[1], (name, us)
+
+
+@pytest.mark.parametrize("group,mode", [(32, 0), (32, 1), (16, 2)])
+def test_fake_quant_of_few_rows(group, mode):
+    """64 and 1000 aligned rows of 128 (an index query's heads) take no longer than unaligned ones, which always go to
+    the row kernel."""
+    from dsv41_amd._lib import call, ptr, stream
+    for n in (64, 1000):
+        x, y = (torch.randn(n * 128 + 2, device=DEV).to(torch.bfloat16) for _ in range(2))
+        us = [_graph_us(lambda a=a, b=b: call("dsv41_fake_quant", ptr(a), ptr(b), n, 128, group, mode, stream(x.device)))
+              for a, b in ((x[:-2], y[:-2]), (x[2:], y[2:]))]
+        assert us[0] <= 1.08 * us[1], us
 
 
 @pytest.mark.parametrize("N,K", [(4096, 5120), (3072, 8192), (4096, 16384), (2048, 16384), (1280, 5120), (300, 64)])

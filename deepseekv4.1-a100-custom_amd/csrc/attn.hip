@@ -1525,6 +1525,9 @@ void plan(int R, int H, int L, int want, int dv, int* nsplit, int* chunk) {
       per = per < 3 ? 3 : per;
       per = per < (tiles + most - 1) / most ? (tiles + most - 1) / most : per;
       if (target == 2 && per < (wgs > 104 ? 12 : 10)) per = tiles;
+      // narrow rows: a tile costs less than the combine (16 rows x 256 keys of 64: one split 12.1 us, three 15.4, of 256
+      // 15.0 and 16.5; 640 keys 20.2 and 16.6, 24.3 and 18.2)
+      if (dv <= 256 && tiles <= 12) per = tiles;
     }
   }
   if (per < 1) per = 1;

@@ -53,3 +53,6 @@ def test_split_plan_of_many_rows():
                              (256, 64, 8320, 1)]:
         n = lib().dsv41_attn_workspace_bytes(R, H, keys, 512, 0)
         assert (n // (R * H * 514 * 4) if n else 1) == want, (R, H, keys)
+    for dv in (64, 128, 256):  # narrow rows, short lists: one split
+        assert lib().dsv41_attn_workspace_bytes(16, 64, 384, dv, 0) == 0
+        assert lib().dsv41_attn_workspace_bytes(16, 64, 416, dv, 0) > 0

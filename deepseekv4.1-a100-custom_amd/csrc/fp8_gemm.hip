@@ -594,9 +594,10 @@ constexpr TileShape kTiles[] = {
     {32, 64, 4, 1, 0.235f, 0.0f, 2.4f},  {32, 128, 4, 1, 0.30f, 0.0f, 2.4f},  {64, 64, 2, 2, 0.30f, 0.48f, 2.0f},
     {64, 128, 1, 2, 0.43f, 0.66f, 2.0f}, {128, 128, 1, 2, 0.62f, 1.05f, 2.5f}};
 constexpr int kTileShapes = sizeof(kTiles) / sizeof(kTiles[0]);
-// Columns up to which the sums stay the streaming kernel's bit for bit: the kv latents (512 columns), whose rows go on
-// to the fp8 grid, where a last bit of a sum becomes a whole step.  Cost at 5120 k, us, against the fastest plan and
-// the stream: 100 rows 11.7 (9.5, 84), 800 23.1 (17.1, 555), 2048 28.6 (25.5, 1425), 3000 46.4 (35.8, 2100).
+// Columns up to which the sums stay the streaming kernel's bit for bit: the kv latents (512 columns), which are cached
+// on the fp8 grid, where a last bit of a sum becomes a whole step.  Wider rows that go on to a grid (the query latents)
+// have sums of the same error in another order.  Cost at 5120 k, us, against the fastest plan and the stream: 100 rows
+// 11.7 (9.5, 84), 800 23.1 (17.1, 555), 2048 28.6 (25.5, 1425), 3000 46.4 (35.8, 2100).
 constexpr int kTileSameN = 512;
 constexpr int kTileMinM = 17;             // up to 16 rows the streaming kernels read the weights once as well
 constexpr long kTilePartMax = 64l << 20;  // bytes of K-slice partials
@@ -705,9 +706,14 @@ long dsv41_fp8_gemm_workspace_bytes(int M, int N, int K) {
   return part ? (long)p.ctiles * 4 + 12 + part : 0;  // counters, pad, partials
 }
 
+int dsv41_fp8_gemm_tile_plan(int M, int N, int K, int group_cols) {
+  if (M <= 0 || N <= 0 || K <= 0 || K % 64 != 0 || !tile_rows_ok(K, group_cols > 0 ? N / group_cols : 1)) return 0;
+  const TilePlan p = tile_plan(M, N, K, group_cols);
+  return p.shape < 0 ? 0 : kTiles[p.shape].bm << 20 | kTiles[p.shape].bn << 10 | p.splits << 1 | p.same;
+}
+
 int dsv41_fp8_gemm_tiled(int M, int N, int K, int group_cols) {
-  return M > 0 && N > 0 && K > 0 && K % 64 == 0 && tile_rows_ok(K, group_cols > 0 ? N / group_cols : 1) &&
-         tile_plan(M, N, K, group_cols).shape >= 0;
+  return dsv41_fp8_gemm_tile_plan(M, N, K, group_cols) != 0;
 }
 
 int dsv41_fp8_gemm(const void* x, long ldx, const void* w8, const void* s8, int M, int N, int K, int Kc,

@@ -53,6 +53,7 @@ SIGNATURES = {
     "dsv41_index_keys_decode": [_P, _P, _L, _P, _P],
     "dsv41_fp8_gemm_workspace_bytes": [_I, _I, _I],
     "dsv41_fp8_gemm_tiled": [_I, _I, _I, _I],
+    "dsv41_fp8_gemm_tile_plan": [_I, _I, _I, _I],
     "dsv41_fp8_gemv_m1_pre": [_P, _P, _F, _I, _P, _P, _I, _I, _I, _P, _P, _L, _P],
     "dsv41_fp8_gemm": [_P, _L, _P, _P, _I, _I, _I, _I, _I, _P, _L, _P, _P, _L, _P],
     "dsv41_f32_proj2": [_P, _L, _P, _P, _I, _I, _I, _P, _P, _P],

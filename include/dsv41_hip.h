@@ -289,8 +289,12 @@ int dsv41_index_keys_decode(const void* k8, const float* ks, long n_rows, void* 
  * once per shape: every launch leaves its arrival counters at zero (launches sharing it must be stream-ordered). */
 long dsv41_fp8_gemm_workspace_bytes(int M, int N, int K);
 
-/* 1 when dsv41_fp8_gemm runs these sizes, with x contiguous and 16-byte aligned, on the tile kernels: their workspace holds no counters, so it needs neither zeroing nor a life beyond the call. */
+/* 1 when dsv41_fp8_gemm runs these sizes, with x contiguous and 16-byte aligned, on the tile kernels: their workspace
+ * holds no counters, so it needs neither zeroing nor a life beyond the call. */
 int dsv41_fp8_gemm_tiled(int M, int N, int K, int group_cols);
+/* The plan of such a launch: 0 where the tile kernels do not apply, else rows << 20 | columns << 10 | K slices << 1 |
+ * (1 when the sums are the streaming kernel's bit for bit). */
+int dsv41_fp8_gemm_tile_plan(int M, int N, int K, int group_cols);
 
 /* fp8_gemm_tc / fp8_gemv_m1 (dsv41/cukern.py:116-200; weight format dsv41/w8.py:19-60): out[m, n] =
  * sum_k x[row(m, n), k] * e4m3(w8[n, k]) * 2^(s8[n / 32, k / 32] - 127), bf16 x (row stride ldx), fp32
@@ -301,7 +305,9 @@ int dsv41_fp8_gemm_tiled(int M, int N, int K, int group_cols);
  * more than 16 rows, K <= 16384) once per up to 128 (the tile kernels).  With x 16-byte aligned and ldx % 8 == 0, up to
  * 16 rows over 1024-4096 columns (up to 4 rows over at most 4096 columns) run without a K split (faster for the decode
  * GEMVs; the workspace is then unused), as does one row there at any alignment of x for K from 512 up to 16384 / 8192 /
- * 5120 / 1280 over up to 1024 / 1536 / 2048 / 4096 columns, or without a workspace. */
+ * 5120 / 1280 over up to 1024 / 1536 / 2048 / 4096 columns, or without a workspace.  Over more than 512 columns the
+ * order of a sum, and with it the last bits of a result, depends on M, on the alignment of x and on whether ws holds
+ * the kernel's K slices; more than 16 rows over up to 512 columns come out the same on either kernel. */
 int dsv41_fp8_gemm(const void* x, long ldx, const void* w8, const void* s8, int M, int N, int K, int Kc,
                    int group_cols, void* out, long ldo, float* out_f32, void* ws, long ws_bytes, void* stream);
 

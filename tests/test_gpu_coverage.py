@@ -58,15 +58,19 @@ def _rope_tables(rd, n):
 # ------------------------------------------------------------------------------------------ many-row attention
 @pytest.mark.parametrize("dqk,R,k,n,nsplit", [(576, 32, 2048, 6000, 0), (576, 48, 300, 250, 0), (512, 24, 512, 9000, 0),
                                               (512, 16, 512, 700, 1), (512, 40, 130, 4000, 3), (512, 300, 100, 99, 0),
-                                              (512, 16, 4100, 6000, 0), (576, 16, 4100, 6000, 0)])
+                                              (512, 16, 4100, 6000, 0), (576, 16, 4100, 6000, 0), (512, 17, 900, 1500, 12),
+                                              (512, 16, 2000, 2500, 67), (576, 16, 2000, 2500, 67), (256, 16, 700, 900, 0),
+                                              (128, 24, 500, 700, 3), (64, 16, 500, 600, 10), (64, 33, 130, 600, 0)])
 def test_sattn2_many_rows_unit_scale(dqk, R, k, n, nsplit):
-    """The 64-head kernel, with (512) and without (576) the inverse rope of the result, at values of unit size against a float64 softmax, three launches bit-equal: gathers still in
-    flight when the output is staged would show in single elements.  Rows end in empty entries as short contexts do.
+    """The 64-head kernel, with (up to 512) and without (576) the inverse rope of the result, up to 67 splits (its
+    combine takes 8 at once, up to 32 and more in three ways), at values of unit size against a float64 softmax, three
+    launches bit-equal: gathers still in flight when the output is staged would show in single elements.  Rows end in
+    empty entries as short contexts do.
     Bound per output row: bf16 probabilities, partials and result round by at most 2^-8, in the 2-norm by under 2^-8.5
     each (independent): sqrt(3) 2^-8.5 < 2^-7."""
     import dsv41_amd
     g = torch.Generator(device=DEV).manual_seed(7)
-    H, dv, win = 64, 512, 128
+    H, dv, win = 64, min(dqk, 512), 128
     rn = lambda *s: torch.randn(*s, generator=g, device=DEV).to(torch.bfloat16)  # noqa: E731
     q, ring, ckv = rn(R, 1, H, dqk), rn(R, win, dqk), rn(R, n, dqk)
     sink = torch.randn(H, generator=g, device=DEV)
@@ -78,7 +82,7 @@ def test_sattn2_many_rows_unit_scale(dqk, R, k, n, nsplit):
     pos = torch.arange(R, device=DEV) + 5000
     seq = torch.arange(R, device=DEV)
     cos, sin = (x.to(DEV) for x in _rope_tables(64, 8192))
-    rd = 64 if dqk == 512 else 0
+    rd = 0 if dqk == 576 else 64
     got = [dsv41_amd.sattn2(q, ring, ckv, idx.unsqueeze(1), pos, sink, cos, sin, rd, dqk ** -0.5, seq, pos, d_v=dv,
                             nsplit=nsplit) for _ in range(3)]
     assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])

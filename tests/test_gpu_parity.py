@@ -1035,17 +1035,28 @@ def test_fp8_gemm_with_the_streaming_kernels_workspace(pad):
     assert torch.equal(out, fp8_gemm_tc(x[:, :K].contiguous(), b, s8))  # (N <= 512: the same bits on both kernels)
 
 
-@pytest.mark.parametrize("M,N,K,gc", [(17, 1280, 5120, 0), (24, 512, 5120, 0), (33, 200, 640, 0), (64, 100, 192, 0),
-                                      (65, 4096, 1280, 0), (100, 4096, 1280, 0), (130, 1024, 512, 128),
-                                      (129, 192, 320, 64), (257, 515, 1280, 0), (300, 2048, 1024, 256),
-                                      (1025, 512, 5120, 0), (2048, 8192, 1024, 0), (2100, 5120, 1024, 0),
-                                      (40, 96, 16384, 0), (20, 64, 16448, 0)])
-def test_fp8_gemm_many_rows(M, N, K, gc):
-    """The tile kernels (more than 16 rows) over their shapes, with and without K slices, row and column remainders and
-    block-diagonal groups, against float64 products of the dequantised weights; the last K runs the streaming kernel.
+@pytest.mark.parametrize("M,N,K,gc,plan", [(17, 1280, 5120, 0, (64, 64, 8, 0)), (24, 512, 5120, 0, (64, 128, 16, 1)),
+    (33, 200, 640, 0, (64, 128, 1, 1)), (64, 100, 192, 0, (64, 128, 1, 1)), (65, 4096, 1280, 0, (32, 64, 1, 0)),
+    (100, 4096, 1280, 0, (32, 64, 1, 0)), (130, 1024, 512, 128, (32, 64, 1, 0)), (129, 192, 320, 64, None),
+    (257, 515, 1280, 0, (32, 64, 1, 0)), (300, 2048, 1024, 256, (64, 64, 1, 0)), (1025, 512, 5120, 0, (64, 64, 1, 1)),
+    (2048, 8192, 1024, 0, (128, 128, 1, 0)), (2100, 5120, 1024, 0, (128, 128, 1, 0)),
+    (40, 96, 16384, 0, (64, 64, 43, 1)), (20, 64, 16448, 0, None), (17, 64, 512, 0, (32, 64, 1, 1)),
+    (33, 64, 8192, 0, (32, 64, 16, 1)), (20, 640, 4096, 0, (32, 64, 8, 0)), (24, 8192, 4096, 1024, (32, 128, 4, 0)),
+    (31, 5000, 8192, 0, (32, 128, 4, 0)), (129, 192, 512, 64, (32, 64, 1, 1)), (100, 8192, 1280, 1024, (64, 64, 1, 0)),
+    (301, 4100, 1280, 0, (64, 128, 1, 0)), (129, 5120, 8192, 0, (64, 128, 4, 0)),
+    (100, 5120, 8192, 0, (128, 128, 4, 0)), (300, 8192, 4096, 1024, (128, 128, 1, 0)),
+    (400, 512, 5120, 0, (128, 128, 20, 1)), (385, 300, 8192, 0, (128, 128, 32, 1))])
+def test_fp8_gemm_many_rows(M, N, K, gc, plan):
+    """The tile kernels (more than 16 rows) over their shapes (plan: rows, columns, K slices, 1 with the streaming
+    kernel's bits; None: the streaming kernel), with and without K slices, row and column remainders and block-diagonal
+    groups, against float64 products of the dequantised weights.
     Bounds: fp32 chains of the streaming kernel's K slices, 1e-5 of the magnitudes (as the other kernels); the bf16 result
     is the fp32 one rounded."""
+    from dsv41_amd._lib import lib
     from dsv41_amd.w8 import W8, fp8_gemm_tc
+    got = lib().dsv41_fp8_gemm_tile_plan(M, N, K, gc)
+    assert (got >> 20, got >> 10 & 1023, got >> 1 & 511, got & 1) == (plan or (0, 0, 0, 0))
+    assert lib().dsv41_fp8_gemm_tiled(M, N, K, gc) == (plan is not None)
     g = torch.Generator(device=DEV).manual_seed(M + N + K)
     b = torch.randint(0, 256, (N, K), generator=g, device=DEV, dtype=torch.uint8)
     b[(b & 0x7F) == 0x7F] = 0x01

@@ -345,7 +345,7 @@ __global__ void __launch_bounds__(kRowThreads) fake_quant_kernel(const uint16_t*
 // flat array, 8 (16 bytes) per lane, a group's maximum taken over its 4 (group 32) or 2 lanes; the values of
 // fake_quant_kernel bit for bit.  The e4m3 grid by the conversion to it and back (v_cvt_pk_fp8_f32 rounds to nearest
 // even); x * rs + 0 gives a negative zero the positive sign round_e4m3 gives it.  3000 rows: 5120 columns fp8
-// 22.2 -> 12.6 us (norm_quant_kernel without a norm), 32 x 128 columns fp4 55.9 -> 12.9 us.
+// 22.2 -> 12.6 us (a thread to a 32-element group), 32 x 128 columns fp4 55.9 -> 12.9 us.
 template <int MODE, int GROUP>
 __global__ void __launch_bounds__(256) fake_quant_flat_kernel(const uint16_t* x, uint16_t* y, long n8) {
   const long e = (long)blockIdx.x * 256 + threadIdx.x;
@@ -410,10 +410,10 @@ __global__ void __launch_bounds__(kRowThreads) rmsnorm_kernel(const uint16_t* x,
   row_op(o, red);
 }
 
-// rmsnorm + per-32 fp8 fake quantisation of rows of up to kNqMaxD elements (dsv41/fused2.py:251-272 norm_quant;
-// without a weight, the fake quantisation alone: dsv41/fused.py:83-84 fake_quant_fp8 on any row length).  Thread t
-// owns the 32-element groups t, t + 256: y = bf16(x * (1 / sqrt(mean(x^2) + eps)) * w), then e4m3 on the group's
-// power-of-two scale, bf16 out.  quant = 0: the rmsnorm alone (dsv41_rmsnorm for rows past the row kernels' 1024).
+// rmsnorm + per-32 fp8 fake quantisation of rows of up to kNqMaxD elements (dsv41/fused2.py:251-272 norm_quant).
+// Thread t owns the 32-element groups t, t + 256: y = bf16(x * (1 / sqrt(mean(x^2) + eps)) * w), then e4m3 on the
+// group's power-of-two scale, bf16 out.  quant = 0: the rmsnorm alone (dsv41_rmsnorm for rows past the row kernels'
+// 1024).
 constexpr int kNqMaxD = 2 * kRowThreads * 32;
 
 __global__ void __launch_bounds__(kRowThreads) norm_quant_kernel(const uint16_t* x, const uint16_t* w, float eps,
@@ -442,16 +442,14 @@ __global__ void __launch_bounds__(kRowThreads) norm_quant_kernel(const uint16_t*
 #pragma unroll
     for (int e = 0; e < 32; ++e) ss += v[q][e] * v[q][e];
   }
-  if (w) {
-    ss = block_sum<kRowThreads>(ss, red);
-    const float inv = __fdiv_rn(1.0f, __fsqrt_rn(__fdiv_rn(ss, (float)D) + eps));
+  ss = block_sum<kRowThreads>(ss, red);
+  const float inv = __fdiv_rn(1.0f, __fsqrt_rn(__fdiv_rn(ss, (float)D) + eps));
 #pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      const int grp = threadIdx.x + kRowThreads * q;
-      if (grp >= ng) break;
+  for (int q = 0; q < 2; ++q) {
+    const int grp = threadIdx.x + kRowThreads * q;
+    if (grp >= ng) break;
 #pragma unroll
-      for (int e = 0; e < 32; ++e) v[q][e] = round_bf16(v[q][e] * inv * bf2f(w[32 * grp + e]));
-    }
+    for (int e = 0; e < 32; ++e) v[q][e] = round_bf16(v[q][e] * inv * bf2f(w[32 * grp + e]));
   }
 #pragma unroll
   for (int q = 0; q < 2; ++q) {

@@ -1394,8 +1394,8 @@ __global__ void __launch_bounds__(256) attn_decode_combine_kernel(const AttnArgs
 }
 
 // Kernel choice: few (row, 64-head) pairs -> decode kernel (16-head workgroups, key splits merged in the launch);
-// otherwise the 64-head kernel, with key splits (bf16 partials + the combine kernel) when the rows alone do not
-// fill the chip.
+// otherwise the 64-head kernel, with key splits (bf16 partials, fp32 ones of rows with the rope inside, and the combine
+// kernel) when the rows alone do not fill the chip.
 // Measured (one layer-step, 576/512, 64 heads, 2176 keys per row): 1 row (C4) decode kernel 18.5 us vs 64-head
 // kernel + splits 30.5 us; 4 rows (C2) 19.8 vs 32.5 us; 48 rows (C5) 85.2 vs 57.3 us (the decode kernel's four
 // 16-head workgroups per row each gather every row: at many rows that redundancy dominates).

@@ -66,9 +66,12 @@ def _indexer_query(x, qrq, wq_b, weights_proj, cos, sin, rd, start_pos, n_heads,
 def compressor_proj(x: torch.Tensor, wkv: torch.Tensor, wgate: torch.Tensor):
     """dsv41/model.py:593-600: the compressor's fp32 projections F.linear(x.float(), wkv), F.linear(x.float(), wgate).
 
-    From 2^20 results a weight on (2048 rows of 512 columns, 5120 k: 120 us against the library's 167; 1500 rows 120
-    to 137, 1000 rows 119 to 98) and in the kernel's form -- bf16 x, fp32 weights of whole 128-column tiles and 64-k stages,
-    contiguous and 16-byte aligned -- by the HIP kernel, otherwise by the library."""
+    From 2^20 results a weight on, which fill half of the card's CUs with the kernel's tiles, and in its form -- bf16 x,
+    fp32 weights of whole 128-column tiles and 64-k stages, contiguous and 16-byte aligned -- by the HIP kernel,
+    otherwise by the library.  Its time is that of one tile up to a tile a CU, the library's grows with the results:
+    2048 rows of 512 columns, 5120 k 123 against 170 us, 256 rows of 4096 122 to 172, 128 of 8192 124 to 167, 17 of
+    65536, 1024 k 135 to 143, 2048 of 512, 64 k 8 to 43.  The two cross under the line (1500 rows of 512 125 to 140, 1000
+    rows 123 to 103), where only 512 columns and 5120 k have been measured."""
     N, K = wkv.shape[0], x.shape[-1]
     M = x.numel() // max(K, 1)
     if (x.is_cuda and M * N >= 1 << 20 and N % 128 == 0 and K % 64 == 0 and K < 1 << 21 and x.dtype == torch.bfloat16
